@@ -72,7 +72,9 @@ struct AttnPlan {
 };
 
 // Plans the split-K launch for an upper bound of dense tokens / blocks.
-AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16);
+// `fewer`: half of the VALU kernel's partial slots, for a caller whose workspace is fixed.
+AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16,
+                   bool fewer = false);
 
 // Enqueues split + merge (+ mean weights / feedback / per-head weights).
 // mean_w: [token count] or null; head_w: [Hq, head_w_ld] or null.

@@ -10,16 +10,12 @@
 //                       cores (tt_attn_mfma.h), grid (splits, Hkv, head
 //                       chunks), 4 waves; one (max, sum, acc[D]) partial per
 //                       (query head, split).
-//   attn_split_kernel   VALU loop, grid (splits, Hkv, head chunks), 4 waves.
-//                       A workgroup owns one KV head and a contiguous, cost-
-//                       balanced range of 16-token tiles: the FP32 tiers (with
-//                       head_dim 128 only these) and, for other head sizes,
-//                       the 2-bit tiles too, unpacked in registers with the
-//                       reference's dequant rounding fmaf(q, scale, zero).
-//                       Lanes are (token group tg = lane/16) x (channel slice
-//                       cp = lane%16); QK partial sums reduce across the 16
-//                       channel lanes of a row with DPP butterflies; online
-//                       softmax over all GQA query heads of the KV head.
+//   attn_split_kernel   VALU loop, grid (splits, Hkv, head chunks), 4 waves:
+//                       head_dim other than 128 (and 64 with an odd number of
+//                       KV heads), FP32 tiers and 2-bit tiles, the latter
+//                       unpacked in registers with the reference's dequant
+//                       rounding fmaf(q, scale, zero); online softmax over all
+//                       GQA query heads of the KV head.
 //   attn_finalize_kernel  LSE merge of the partials -> attn_output, and in the
 //                       same launch the mean attention weights over query
 //                       heads (:286-300), optional per-head weights and the
@@ -55,8 +51,6 @@ __device__ __forceinline__ float row_sum16(float x) {
     return x;
 }
 
-__device__ __forceinline__ float shfl_xor(float x, int m) { return __shfl_xor(x, m, 64); }
-
 template <int N>
 __device__ __forceinline__ void load_f32(const float* __restrict__ p, float (&x)[N]) {
     if constexpr (N % 4 == 0) {
@@ -77,49 +71,6 @@ __device__ __forceinline__ void load_f32(const float* __restrict__ p, float (&x)
     }
 }
 
-template <int N>
-__device__ __forceinline__ void load_u32(const int32_t* __restrict__ p, uint32_t (&x)[N]) {
-    if constexpr (N % 4 == 0) {
-#pragma unroll
-        for (int j = 0; j < N; j += 4) {
-            const int4 v = *reinterpret_cast<const int4*>(p + j);
-            x[j] = v.x; x[j + 1] = v.y; x[j + 2] = v.z; x[j + 3] = v.w;
-        }
-    } else if constexpr (N % 2 == 0) {
-#pragma unroll
-        for (int j = 0; j < N; j += 2) {
-            const int2 v = *reinterpret_cast<const int2*>(p + j);
-            x[j] = v.x; x[j + 1] = v.y;
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j) x[j] = static_cast<uint32_t>(p[j]);
-    }
-}
-
-template <typename MetaT, int N>
-__device__ __forceinline__ void load_meta(const MetaT* __restrict__ p, float (&x)[N]) {
-    if constexpr (sizeof(MetaT) == 4) {
-        load_f32<N>(reinterpret_cast<const float*>(p), x);
-    } else {
-        if constexpr (N % 8 == 0) {
-#pragma unroll
-            for (int j = 0; j < N; j += 8) {
-                const uint4 v = *reinterpret_cast<const uint4*>(p + j);
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    x[j + 2 * k] = f16_to_f32(static_cast<uint16_t>(w[k] & 0xffffu));
-                    x[j + 2 * k + 1] = f16_to_f32(static_cast<uint16_t>(w[k] >> 16));
-                }
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < N; ++j) x[j] = f16_to_f32(reinterpret_cast<const uint16_t*>(p)[j]);
-        }
-    }
-}
-
 struct SplitArgs {
     AttnInputs in;
     float scale2;  // log2(e) / sqrt(head_dim): logits are kept in log2 units
@@ -130,67 +81,175 @@ struct SplitArgs {
     int nsplit;      // partial slots per query head
     int nsplit_p;    // matrix-core workgroups over the packed store: slots [0, nsplit_p)
     int nsplit_d;    // VALU workgroups: slots [nsplit_p, nsplit)
-    int wd, wp;      // tile cost weights: dense, packed
     int dense_delay; // FP32-tier workgroups wait this many 10 ns ticks before their first tile load
 };
 
-// LDS of the VALU tile loop: per-wave (max, sum, acc[D]) for the final merge.
-template <int D, int GP>
+#include "tt_attn_mfma.h"
+
+// ---------------------------------------------------------------------------
+// The VALU loop (head_dim other than 128, and 64 with an odd number of KV
+// heads). FP32 arithmetic throughout: operands, products and sums.
+// ---------------------------------------------------------------------------
+
+// Tokens of one FP32 unit of a wave: half a tile for the head dims whose rows of four tokens per lane would take
+// 128 registers.
+__host__ __device__ constexpr int split_unit_tokens(const int D) { return D > 128 ? 8 : 16; }
+
+// Floats of one (value, row group) line in the merge area: 16 channel lanes and one of padding.
+constexpr int kSplitLine = 17;
+
+// LDS of the VALU tile loop: per wave the accumulators and the sums of its
+// heads, reduced over the wave's row groups, and its maxima.
+template <int CPL, int GP>
 struct SplitLds {
-    static constexpr int BYTES = 4 * GP * (2 + D) * 4;
+    static constexpr int VALUES = (GP * (CPL + 1) + 3) / 4 * 4;  // GP x CPL accumulators, GP sums, padding
+    static constexpr int BYTES = 4 * (VALUES * kSplitLine + GP) * 4;
 };
+
+// N consecutive words, floats or metadata entries in as few loads as their
+// count allows. They need be aligned to an entry only (a head's row starts at
+// a multiple of head_dim entries, a lane's slice at a multiple of head_dim /
+// 16): the types say two bytes, and the hardware takes any.
+template <int N>
+__device__ __forceinline__ void load_slice(const uint32_t* __restrict__ p, uint32_t (&x)[N]) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(2)));
+    typedef uint32_t u2 __attribute__((ext_vector_type(2), aligned(2)));
+    typedef uint32_t u1 __attribute__((aligned(2)));
+    constexpr int N4 = N / 4 * 4;
+#pragma unroll
+    for (int j = 0; j < N4; j += 4) {
+        const u4 v = *reinterpret_cast<const u4*>(p + j);
+        x[j] = v.x; x[j + 1] = v.y; x[j + 2] = v.z; x[j + 3] = v.w;
+    }
+    if constexpr (N - N4 >= 2) {
+        const u2 v = *reinterpret_cast<const u2*>(p + N4);
+        x[N4] = v.x; x[N4 + 1] = v.y;
+    }
+    if constexpr ((N - N4) % 2 == 1) x[N - 1] = *reinterpret_cast<const u1*>(p + N - 1);
+}
+template <int N>
+__device__ __forceinline__ void load_slice(const float* __restrict__ p, float (&x)[N]) {
+    uint32_t u[N];
+    load_slice<N>(reinterpret_cast<const uint32_t*>(p), u);
+#pragma unroll
+    for (int j = 0; j < N; ++j) x[j] = __uint_as_float(u[j]);
+}
+// Metadata of a lane's slice in its stored width, converted where it is used.
+template <typename MetaT, int N>
+struct MetaSlice;
+template <int N>
+struct MetaSlice<float, N> {
+    float v[N];
+    __device__ __forceinline__ void load(const float* __restrict__ p) { load_slice<N>(p, v); }
+    __device__ __forceinline__ float get(const int j) const { return v[j]; }
+};
+template <int N>
+struct MetaSlice<uint16_t, N> {
+    static constexpr bool kPairs = N % 2 == 0;  // read two entries per word
+    uint32_t v[kPairs ? N / 2 : N];
+    __device__ __forceinline__ void load(const uint16_t* __restrict__ p) {
+        if constexpr (kPairs) {
+            load_slice<N / 2>(reinterpret_cast<const uint32_t*>(p), v);
+        } else {
+#pragma unroll
+            for (int j = 0; j < N; ++j) v[j] = p[j];
+        }
+    }
+    __device__ __forceinline__ float get(const int j) const {
+        if constexpr (kPairs)
+            return f16_to_f32(static_cast<uint16_t>((j & 1) ? v[j / 2] >> 16 : v[j / 2] & 0xffffu));
+        else
+            return f16_to_f32(static_cast<uint16_t>(v[j]));
+    }
+};
+
+__device__ __forceinline__ float meta_value(const float v) { return v; }
+__device__ __forceinline__ float meta_value(const uint16_t v) { return f16_to_f32(v); }
+
+// The codes at bits 0, 8, 16 and 24 of x, each alone in its byte, from where
+// one conversion makes a float of it. (Opaque, or the compiler extracts every
+// code with an instruction of its own and converts it from byte 0.)
+__device__ __forceinline__ uint32_t code_bytes(const uint32_t x) {
+    uint32_t y = x & 0x03030303u;
+    asm("" : "+v"(y));
+    return y;
+}
+
+// Sum over the four 16-lane rows of four values at once: row r of the result
+// holds the total of v[r] (two swaps that exchange half of the rows, an add
+// after each).
+__device__ __forceinline__ float rows_sum4(const float (&v)[4]) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]), __float_as_uint(v[1]), false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[2]), __float_as_uint(v[3]), false, false);
+    const float x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const float y = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(c[0]) + __uint_as_float(c[1]);
+}
 
 // CPL: channels per lane (head_dim / 16). GP: query heads per workgroup
 // (padded to a power of two; heads past the group are zero and never stored).
+//
+// Each wave owns a contiguous share of its KV head's units: FP32 units of
+// split_unit_tokens, then 16-token packed tiles, counted alike (an FP32 unit
+// holds more bytes and needs fewer instructions; at two, four or eight tiles
+// per FP32 unit the launches took the same or up to 15% longer). Share
+// wave nsplit_d + split, so that every workgroup holds both kinds. Lane (row group tg, channel lane cp) holds channels
+// cp CPL .. + CPL - 1 of tokens tg, tg + 4, ...: a K word shifted by 2 tg has
+// those tokens' codes in the low bits of its four bytes, so one mask and four
+// byte conversions unpack them. The row's logits come from a DPP sum over its
+// 16 lanes; V is unpacked after the softmax, when K is no longer live.
+//
+// A wave has one to three units, so the launch is a chain: arguments, query
+// and first unit's loads, arithmetic (about 850 VALU instructions per packed
+// tile at head_dim 256 with two heads, 350 at head_dim 80 with one), the next
+// unit, the merge. What it responds to is the length of that chain: 32-bit
+// shares of the work (64-bit divides took about 2 us), loads as wide as the
+// row allows from scalar bases, and registers for three to six waves per SIMD.
+// Partials per launch: head_dim 256 with 16/8 heads at 8k 18.7 -> 11.6 us,
+// head_dim 80 with 32/32 heads at 2k 10.3 -> 6.2, head_dim 96 with 32/32
+// heads at 4k 15.2 -> 9.1, head_dim 64 with 9/3 heads at 8k 9.4 -> 6.4.
 template <int CPL, int GP, typename MetaT>
 __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, char* lds) {
     constexpr int D = 16 * CPL;
+    constexpr int NTD = split_unit_tokens(D) / 4;  // FP32 tokens per lane and unit
     const AttnInputs& in = a.in;
     const int kvh = blockIdx.y;
     const int G = in.Hq / in.Hkv;
     const int g0 = blockIdx.z * GP;
     const int gc = min(GP, G - g0);
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tg = lane >> 4;
     const int cp = lane & 15;
-
-    int n0 = in.n0, n1 = in.n1, n2 = in.n2, head = in.ring_head, nb = in.num_blocks;
-    if (in.state) {
-        n0 = in.state[kSCount];
-        n1 = in.state[kHhCount];
-        n2 = in.state[kRwCount];
-        head = in.state[kRwHead];
-        nb = in.state[kBlocksUsed];
-    }
-    const int Nd = n0 + n1 + n2;
-    const int W = in.kgs >> 4;
-    const int Td = (Nd + 15) >> 4;
-    const int Tp = nb * W;
-    const int Hkv = in.Hkv;
-
-    // Cost-balanced contiguous tile range of this split.
-    const long long U = static_cast<long long>(Td) * a.wd + static_cast<long long>(Tp) * a.wp;
-    const long long lo = U * split / a.nsplit_d, hi = U * (split + 1) / a.nsplit_d;
-    auto cdiv = [](long long x, long long y) -> long long { return x <= 0 ? 0 : (x + y - 1) / y; };
-    const int d_begin = static_cast<int>(min(cdiv(lo, a.wd), static_cast<long long>(Td)));
-    const int d_end = static_cast<int>(min(cdiv(hi, a.wd), static_cast<long long>(Td)));
-    const long long pb = static_cast<long long>(Td) * a.wd;
-    const int p_begin = static_cast<int>(min(cdiv(lo - pb, a.wp), static_cast<long long>(Tp)));
-    const int p_end = static_cast<int>(min(cdiv(hi - pb, a.wp), static_cast<long long>(Tp)));
-    const int nd = d_end - d_begin;
-    const int nt = nd + (p_end - p_begin);
 
     float q[GP][CPL];
 #pragma unroll
     for (int g = 0; g < GP; ++g) {
-        if (g < gc) {
-            load_f32<CPL>(in.Q + static_cast<size_t>(kvh * G + g0 + g) * D + cp * CPL, q[g]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < CPL; ++j) q[g][j] = 0.0f;
-        }
+        // heads past the group repeat its last one (their results are not stored)
+        load_slice<CPL>(in.Q + static_cast<size_t>(kvh * G + g0 + min(g, gc - 1)) * D + cp * CPL, q[g]);
     }
+
+    int n0 = in.n0, n1 = in.n1, n2 = in.n2, head = in.ring_head, nb = in.num_blocks;
+    auto uniform = [](const int x) { return __builtin_amdgcn_readfirstlane(x); };
+    if (in.state) {
+        n0 = uniform(in.state[kSCount]);
+        n1 = uniform(in.state[kHhCount]);
+        n2 = uniform(in.state[kRwCount]);
+        head = uniform(in.state[kRwHead]);
+        nb = uniform(in.state[kBlocksUsed]);
+    }
+    const int Nd = n0 + n1 + n2;
+    const int W = in.kgs >> 4;
+    const int Td = (Nd + 4 * NTD - 1) / (4 * NTD);
+    const int Tp = nb * W;
+    const int Hkv = in.Hkv;
+
+    // The wave's share of the Td FP32 units and Tp packed tiles.
+        const int part = wave * a.nsplit_d + split, parts = 4 * a.nsplit_d;
+    const int lo = part_begin(Td + Tp, part, parts), hi = part_begin(Td + Tp, part + 1, parts);
+    const int d_begin = min(lo, Td), d_end = min(hi, Td);
+    const int p_begin = max(lo - Td, 0), p_end = max(hi - Td, 0);
 
     float m[GP], l[GP], acc[GP][CPL];
 #pragma unroll
@@ -201,183 +260,206 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
         for (int j = 0; j < CPL; ++j) acc[g][j] = 0.0f;
     }
 
+    // Lane cp = NT (g % HS) + i stores the logit of head g, token tok0 + tg + 4 i.
+    auto put_logits = [&](const auto& s, const int tok0, const int limit) {
+        constexpr int NT = sizeof(s) / sizeof(s[0]);
+        constexpr int HS = 16 / NT < GP ? 16 / NT : GP;  // heads per store
+#pragma unroll
+        for (int h0 = 0; h0 < GP; h0 += HS) {
+            float v = s[0][h0];
+#pragma unroll
+            for (int g = 0; g < HS; ++g)
+#pragma unroll
+                for (int i = 0; i < NT; ++i) v = (cp == NT * g + i) ? s[i][h0 + g] : v;
+            const int g = h0 + cp / NT, t = tok0 + tg + 4 * (cp % NT);
+            if (cp < NT * HS && g < gc && t < limit)
+                st_dev1(a.logits + static_cast<size_t>(kvh * G + g0 + g) * a.ld + t, v);
+        }
+    };
+    // Online softmax: logits to weights, the accumulators to the new maximum
+    // (exact, and the same in every lane).
+    auto softmax = [&](auto& s) {
+        constexpr int NT = sizeof(s) / sizeof(s[0]);
+#pragma unroll
+        for (int g = 0; g < GP; ++g) {
+            float tm = s[0][g];
+#pragma unroll
+            for (int i = 1; i < NT; ++i) tm = fmax_nn(tm, s[i][g]);
+            const float mn = fmax_nn(m[g], xrow_max(tm));
+            const float alpha = (m[g] == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(m[g] - mn);
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                s[i][g] = (s[i][g] == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(s[i][g] - mn);
+                sum += s[i][g];
+            }
+            l[g] = __builtin_fmaf(l[g], alpha, sum);
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) acc[g][j] *= alpha;
+            m[g] = mn;
+        }
+    };
+
+#pragma unroll 1
+    for (int k = d_begin; k < d_end; ++k) {
+        // ---- FP32 unit: logical rows 4 NTD k ... ----
+        const int tok0 = 4 * NTD * k;
+        float kx[NTD][CPL], vx[NTD][CPL];
+        size_t off[NTD];
+        const float* vb[NTD];
+#pragma unroll
+        for (int i = 0; i < NTD; ++i) {
+            const int r = min(tok0 + tg + 4 * i, Nd - 1);  // rows past the tiers are masked below
+            const bool in0 = r < n0, in1 = r < n0 + n1;
+            int ring = head + (r - n0 - n1);
+            ring = ring >= in.ring_size ? ring - in.ring_size : ring;
+            const int idx = in0 ? r : (in1 ? r - n0 : ring);
+            off[i] = (static_cast<size_t>(idx) * Hkv + kvh) * D + cp * CPL;
+            vb[i] = in0 ? in.v0 : (in1 ? in.v1 : in.v2);
+            load_slice<CPL>((in0 ? in.k0 : (in1 ? in.k1 : in.k2)) + off[i], kx[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NTD; ++i) load_slice<CPL>(vb[i] + off[i], vx[i]);
+        float s[NTD][GP];
+#pragma unroll
+        for (int i = 0; i < NTD; ++i)
+#pragma unroll
+            for (int g = 0; g < GP; ++g) {
+                float d = 0.0f;
+#pragma unroll
+                for (int j = 0; j < CPL; ++j) d = __builtin_fmaf(q[g][j], kx[i][j], d);
+                d = row_sum16(d) * a.scale2;
+                s[i][g] = (tok0 + tg + 4 * i < Nd) ? d : kNegInf;
+            }
+        if (a.logits) put_logits(s, tok0, Nd);
+        softmax(s);
+#pragma unroll
+        for (int i = 0; i < NTD; ++i)
+#pragma unroll
+            for (int g = 0; g < GP; ++g)
+#pragma unroll
+                for (int j = 0; j < CPL; ++j) acc[g][j] = __builtin_fmaf(s[i][g], vx[i][j], acc[g][j]);
+    }
+
     const MetaT* ks = static_cast<const MetaT*>(in.ks);
     const MetaT* kz = static_cast<const MetaT*>(in.kz);
     const MetaT* vs = static_cast<const MetaT*>(in.vs);
     const MetaT* vz = static_cast<const MetaT*>(in.vz);
+    // The lane's CPL channels are 2 CPL bits of the row's code words, from bit
+    // 2 (c0 % 16) of word c0 / 16 on (in two words where CPL does not divide 16).
+    constexpr bool kOneWord = (16 % CPL) == 0;
+    const int c0 = cp * CPL;
+    const int cw = c0 >> 4, csh = 2 * (c0 & 15);
+    const int cw1 = min(cw + 1, CPL - 1);
+    // Loads take a wave-uniform base and a 32-bit lane offset: K words and
+    // metadata from the tile's (block's) row, V words and metadata from the
+    // rows of tokens 4 i, at the same lane offset for every i. (The offset is
+    // opaque, or its 64-bit extension is hoisted out of the loop and every
+    // load takes a 64-bit vector add instead of the scalar base.)
+    auto at = [](const void* base, uint32_t off) {
+        asm("" : "+v"(off));
+        return static_cast<const char*>(base) + off;
+    };
+    const uint32_t k_off = static_cast<uint32_t>(kvh * D + c0);
+    const uint32_t v_row = static_cast<uint32_t>(tg * Hkv + kvh);
+    const uint32_t v_off = (v_row * CPL + cw) * 4u, v_off1 = (v_row * CPL + cw1) * 4u;
 
-    for (int it = wave; it < nt; it += 4) {
-        float s[4][GP];
-        float vx[4][CPL];
-        bool valid[4];
-        int tok0;  // logical index of token 0 of this lane's row group
-        if (it < nd) {
-            // ---- FP32 dense tile: logical rows 16k .. 16k+15 ----
-            const int k = d_begin + it;
-            tok0 = 16 * k + 4 * tg;
-            float kx[4][CPL];
+#pragma unroll 1
+    for (int t = p_begin; t < p_end; ++t) {
+        // ---- 2-bit packed tile: half (kgs 32) or whole (kgs 16) block ----
+        // (an opaque copy of the index: the compiler would keep an address per
+        // load in registers over the loop, about 30 in all)
+        int kt = t;
+        asm("" : "+s"(kt));
+        const size_t krow = static_cast<size_t>(kt) * Hkv * D;
+        const size_t mrow = static_cast<size_t>(W == 2 ? kt >> 1 : kt) * Hkv * D;
+        const size_t slot0 = static_cast<size_t>(16) * kt;
+        const long long id = *reinterpret_cast<const long long*>(at(in.ids + slot0, 8u * cp));
+        uint32_t kw[CPL];
+        MetaSlice<MetaT, CPL> ksc, kze;
+        load_slice<CPL>(reinterpret_cast<const uint32_t*>(at(in.kp + krow, 4u * k_off)), kw);
+        ksc.load(reinterpret_cast<const MetaT*>(at(ks + mrow, sizeof(MetaT) * k_off)));
+        kze.load(reinterpret_cast<const MetaT*>(at(kz + mrow, sizeof(MetaT) * k_off)));
+        uint32_t vw[4], vw1[4];
+        MetaT vsr[4], vzr[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int r = tok0 + i;
-                valid[i] = r < Nd;
-                if (valid[i]) {
-                    const float* kb;
-                    const float* vb;
-                    int idx;
-                    if (r < n0) {
-                        kb = in.k0; vb = in.v0; idx = r;
-                    } else if (r < n0 + n1) {
-                        kb = in.k1; vb = in.v1; idx = r - n0;
-                    } else {
-                        kb = in.k2; vb = in.v2;
-                        idx = head + (r - n0 - n1);
-                        if (idx >= in.ring_size) idx -= in.ring_size;
-                    }
-                    const size_t off = (static_cast<size_t>(idx) * Hkv + kvh) * D + cp * CPL;
-                    load_f32<CPL>(kb + off, kx[i]);
-                    load_f32<CPL>(vb + off, vx[i]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < CPL; ++j) { kx[i][j] = 0.0f; vx[i][j] = 0.0f; }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int g = 0; g < GP; ++g) {
-                    float d = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < CPL; ++j) d = __builtin_fmaf(q[g][j], kx[i][j], d);
-                    s[i][g] = d;
-                }
-        } else {
-            // ---- 2-bit packed tile: half (kgs 32) or whole (kgs 16) block ----
-            const int kt = p_begin + (it - nd);
-            const int b = kt / W, w = kt - b * W;
-            const int slot0 = b * in.kgs + w * 16 + 4 * tg;
-            tok0 = Nd + slot0;
-            uint32_t kw[CPL];
-            float ksc[CPL], kze[CPL];
-            load_u32<CPL>(in.kp + ((static_cast<size_t>(b) * W + w) * Hkv + kvh) * D + cp * CPL, kw);
-            const size_t moff = (static_cast<size_t>(b) * Hkv + kvh) * D + cp * CPL;
-            load_meta<MetaT, CPL>(ks + moff, ksc);
-            load_meta<MetaT, CPL>(kz + moff, kze);
-            const longlong2 id01 = *reinterpret_cast<const longlong2*>(in.ids + slot0);
-            const longlong2 id23 = *reinterpret_cast<const longlong2*>(in.ids + slot0 + 2);
-            valid[0] = id01.x != -1; valid[1] = id01.y != -1;
-            valid[2] = id23.x != -1; valid[3] = id23.y != -1;
-            const int qhd = D / 16;
-            // The lane's channels c0 .. c0 + CPL - 1 lie in V word c0 / 16, and
-            // in the next word too when CPL does not divide 16 (head_dim 48,
-            // 80, 96, ...; CPL <= 16, so never a third).
-            constexpr bool kOneWord = (16 % CPL) == 0;
-            const int c0 = cp * CPL;
-            const int cw = c0 >> 4;
-            const int cw1 = kOneWord ? cw : ((c0 + CPL - 1) >> 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = 4 * tg + i;  // token within the 16-token word
-                const size_t vrow = static_cast<size_t>(slot0 + i) * Hkv + kvh;
-                const uint32_t vwd = static_cast<uint32_t>(in.vp[vrow * qhd + cw]);
-                const uint32_t vwd1 = kOneWord ? vwd : static_cast<uint32_t>(in.vp[vrow * qhd + cw1]);
-                const float vsc = Meta<MetaT>::load(vs, vrow);
-                const float vze = Meta<MetaT>::load(vz, vrow);
-#pragma unroll
-                for (int j = 0; j < CPL; ++j) {
-                    const int c = c0 + j;
-                    const uint32_t w = (kOneWord || (c >> 4) == cw) ? vwd : vwd1;
-                    vx[i][j] = __builtin_fmaf(static_cast<float>((w >> (2 * (c & 15))) & 3u), vsc, vze);
-                }
-                float kd[CPL];
-#pragma unroll
-                for (int j = 0; j < CPL; ++j)
-                    kd[j] = __builtin_fmaf(static_cast<float>((kw[j] >> (2 * t)) & 3u), ksc[j], kze[j]);
-#pragma unroll
-                for (int g = 0; g < GP; ++g) {
-                    float d = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < CPL; ++j) d = __builtin_fmaf(q[g][j], kd[j], d);
-                    s[i][g] = d;
-                }
-            }
+        for (int i = 0; i < 4; ++i) {
+            const size_t row = (slot0 + 4 * i) * Hkv;
+            vw[i] = *reinterpret_cast<const uint32_t*>(at(in.vp + row * CPL, v_off));
+            vw1[i] = kOneWord ? 0u : *reinterpret_cast<const uint32_t*>(at(in.vp + row * CPL, v_off1));
+            vsr[i] = *reinterpret_cast<const MetaT*>(at(vs + row, sizeof(MetaT) * v_row));
+            vzr[i] = *reinterpret_cast<const MetaT*>(at(vz + row, sizeof(MetaT) * v_row));
         }
-
-        // QK partial sums -> full dot products (every lane of the row).
+        float s[4][GP];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int g = 0; g < GP; ++g) {
-                const float d = row_sum16(s[i][g]) * a.scale2;
-                s[i][g] = valid[i] ? d : kNegInf;
-            }
-
-        if (a.logits) {
-#pragma unroll
-            for (int g = 0; g < GP; ++g) {
-                if (g < gc && cp == g) {
-                    float* lr = a.logits + static_cast<size_t>(kvh * G + g0 + g) * a.ld;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (it >= nd || tok0 + i < Nd) lr[tok0 + i] = s[i][g];
-                }
-            }
-        }
-
-        // Online softmax update (max is exact, so every lane agrees on m).
-#pragma unroll
-        for (int g = 0; g < GP; ++g) {
-            float tm = fmaxf(fmaxf(s[0][g], s[1][g]), fmaxf(s[2][g], s[3][g]));
-            tm = fmaxf(tm, shfl_xor(tm, 16));
-            tm = fmaxf(tm, shfl_xor(tm, 32));
-            const float mn = fmaxf(m[g], tm);
-            const float alpha = (m[g] == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(m[g] - mn);
-            float p[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) p[i] = (s[i][g] == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(s[i][g] - mn);
-            l[g] = __builtin_fmaf(l[g], alpha, (p[0] + p[1]) + (p[2] + p[3]));
-#pragma unroll
-            for (int j = 0; j < CPL; ++j) {
-                float v = acc[g][j] * alpha;
-                v = __builtin_fmaf(p[0], vx[0][j], v);
-                v = __builtin_fmaf(p[1], vx[1][j], v);
-                v = __builtin_fmaf(p[2], vx[2][j], v);
-                v = __builtin_fmaf(p[3], vx[3][j], v);
-                acc[g][j] = v;
-            }
-            m[g] = mn;
-        }
-    }
-
-    // Reduce the four row groups (each accumulated its own tokens).
-#pragma unroll
-    for (int g = 0; g < GP; ++g) {
-        l[g] += shfl_xor(l[g], 16);
-        l[g] += shfl_xor(l[g], 32);
+            for (int g = 0; g < GP; ++g) s[i][g] = 0.0f;
 #pragma unroll
         for (int j = 0; j < CPL; ++j) {
-            acc[g][j] += shfl_xor(acc[g][j], 16);
-            acc[g][j] += shfl_xor(acc[g][j], 32);
+            const uint32_t x = code_bytes(kw[j] >> (2 * tg));
+            const float sc = ksc.get(j), ze = kze.get(j);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float kd = __builtin_fmaf(static_cast<float>((x >> (8 * i)) & 0xffu), sc, ze);
+#pragma unroll
+                for (int g = 0; g < GP; ++g) s[i][g] = __builtin_fmaf(q[g][j], kd, s[i][g]);
+            }
+        }
+        const unsigned valid = static_cast<unsigned>(__ballot(id != -1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool ok = (valid >> (tg + 4 * i)) & 1u;
+#pragma unroll
+            for (int g = 0; g < GP; ++g) {
+                const float d = row_sum16(s[i][g]) * a.scale2;
+                s[i][g] = ok ? d : kNegInf;
+            }
+        }
+        if (a.logits) put_logits(s, Nd + 16 * kt, Nd + 16 * kt + 16);
+        softmax(s);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t w = kOneWord ? vw[i] >> csh : __builtin_amdgcn_alignbit(vw1[i], vw[i], csh);
+            const float vsc = meta_value(vsr[i]), vze = meta_value(vzr[i]);
+            // channel 4 b + k in byte b of word k (fewer than eight channels: the codes one by one)
+            uint32_t wk[4];
+            if constexpr (CPL >= 8) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) wk[k] = code_bytes(w >> (2 * k));
+            }
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const uint32_t c = CPL >= 8 ? (wk[j & 3] >> (8 * (j >> 2))) & 0xffu : (w >> (2 * j)) & 3u;
+                const float v = __builtin_fmaf(static_cast<float>(c), vsc, vze);
+#pragma unroll
+                for (int g = 0; g < GP; ++g) acc[g][j] = __builtin_fmaf(s[i][g], v, acc[g][j]);
+            }
         }
     }
 
-    // Merge the four waves in LDS and store one partial per query head.
-    float* sm_m = reinterpret_cast<float*>(lds);  // [4][GP]
-    float* sm_l = sm_m + 4 * GP;                   // [4][GP]
-    float* sm_acc = sm_l + 4 * GP;                 // [4][GP][D]
-    if (tg == 0) {
+    // Reduce the four row groups (each accumulated its own tokens), four
+    // values at a time, then merge the four waves in LDS and store one partial
+    // per query head.
+    constexpr int NV = SplitLds<CPL, GP>::VALUES;
+    float* sm = reinterpret_cast<float*>(lds);  // [4 waves][NV][kSplitLine]
+    float* sm_m = sm + 4 * NV * kSplitLine;     // [4][GP]
+    auto value = [&](const int v) {
+        return v < GP * CPL ? acc[v / CPL][v % CPL] : (v < GP * (CPL + 1) ? l[v - GP * CPL] : 0.0f);
+    };
 #pragma unroll
-        for (int g = 0; g < GP; ++g) {
+    for (int v = 0; v < NV; v += 4) {
+        const float x[4] = {value(v), value(v + 1), value(v + 2), value(v + 3)};
+        sm[(wave * NV + v + tg) * kSplitLine + cp] = rows_sum4(x);
+    }
+    if (lane == 0) {
 #pragma unroll
-            for (int j = 0; j < CPL; ++j) sm_acc[(wave * GP + g) * D + cp * CPL + j] = acc[g][j];
-            if (cp == 0) {
-                sm_m[wave * GP + g] = m[g];
-                sm_l[wave * GP + g] = l[g];
-            }
-        }
+        for (int g = 0; g < GP; ++g) sm_m[wave * GP + g] = m[g];
     }
     __syncthreads();
     for (int idx = threadIdx.x; idx < gc * D; idx += 256) {
         const int g = idx / D, c = idx - g * D;
+        const int line = g * CPL + c % CPL, col = c / CPL;
         float M = kNegInf;
 #pragma unroll
         for (int w = 0; w < 4; ++w) M = fmaxf(M, sm_m[w * GP + g]);
@@ -387,26 +469,24 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
             for (int w = 0; w < 4; ++w) {
                 const float mw = sm_m[w * GP + g];
                 const float f = (mw == kNegInf) ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
-                A = __builtin_fmaf(f, sm_acc[(w * GP + g) * D + c], A);
-                L = __builtin_fmaf(f, sm_l[w * GP + g], L);
+                A = __builtin_fmaf(f, sm[(w * NV + line) * kSplitLine + col], A);
+                L = __builtin_fmaf(f, sm[(w * NV + GP * CPL + g) * kSplitLine], L);
             }
         }
         const size_t pi = static_cast<size_t>(kvh * G + g0 + g) * a.nsplit + a.nsplit_p + split;
-        a.part_acc[pi * D + c] = A;
+        st_dev1(a.part_acc + pi * D + c, A);
         if (c == 0) {
-            a.part_ml[2 * pi] = M;
-            a.part_ml[2 * pi + 1] = L;
+            st_dev1(a.part_ml + 2 * pi, M);
+            st_dev1(a.part_ml + 2 * pi + 1, L);
         }
     }
 }
 
 template <int CPL, int GP, typename MetaT>
 __global__ void __launch_bounds__(256) attn_split_kernel(SplitArgs a) {
-    __shared__ __align__(16) char lds[SplitLds<16 * CPL, GP>::BYTES];
+    __shared__ __align__(16) char lds[SplitLds<CPL, GP>::BYTES];
     split_body<CPL, GP, MetaT>(a, static_cast<int>(blockIdx.x), lds);
 }
-
-#include "tt_attn_mfma.h"
 
 // head_dim 128: a 1-D grid of ceil(nsplit / 8) * 8 slots per (KV head, head
 // chunk). Slots s < nsplit_p run the matrix-core loop over pair range s of
@@ -1034,8 +1114,6 @@ attn_batched_kernel(const BatchArgs b) {
     a.nsplit = b.slot_base[i + 1] - b.slot_base[i];
     a.nsplit_p = b.pk_base[i + 1] - b.pk_base[i];
     a.nsplit_d = a.nsplit - a.nsplit_p;
-    a.wd = 8;
-    a.wp = 1;
     a.dense_delay = 0;
     const int kvh = hz / b.chunks, chunk = hz - kvh * b.chunks;
     if (s >= a.nsplit_p) {
@@ -1272,7 +1350,7 @@ int attn_check_shapes(int Hq, int Hkv, int D, int kgs) {
 
 namespace {
 AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                        int meta_fp16, bool pair);
+                        int meta_fp16, bool pair, bool fewer);
 }  // namespace
 
 // Head_dim 64 with an even number of KV heads runs as half as many heads of
@@ -1281,18 +1359,19 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
 // token, FP32 rows), so they read like one head of 128 channels, and the
 // query heads of both form one group whose queries fill the half of their own
 // head (zeros in the other half), which leaves their logits exact.
-AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16) {
+AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16,
+                   bool fewer) {
     if (D == 64 && Hkv % 2 == 0) {
-        AttnPlan p = attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv / 2, kMfD, kgs, need_logits, meta_fp16, true);
+        AttnPlan p = attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv / 2, kMfD, kgs, need_logits, meta_fp16, true, fewer);
         p.pair64 = true;
         return p;
     }
-    return attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv, D, kgs, need_logits, meta_fp16, false);
+    return attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv, D, kgs, need_logits, meta_fp16, false, fewer);
 }
 
 namespace {
 AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                        int meta_fp16, bool pair) {
+                        int meta_fp16, bool pair, bool fewer) {
     AttnPlan p;
     const int W = kgs / 16;
     const int G = Hq / Hkv;
@@ -1381,21 +1460,27 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
             p.dense_delay = static_cast<int>(std::min<long long>(550, burst / 19000));
         }
     } else {
-        // One round of resident workgroups, two when four or more fit on a
-        // CU (head_dim up to ~128 at one or two heads per group), with at
-        // least ~8 packed-tile units of work per workgroup and round: the
-        // loop is arithmetic-bound, and fewer, longer workgroups left CUs
-        // idle. Per launch: head_dim 256 with 16/8 heads at 8k context (two
-        // workgroups per CU) 20.9 us against 35.9 with ~32 units per
-        // workgroup and 24.6 with two rounds; head_dim 80 with 32/32 heads at
-        // 2k (five per CU) 11.2 against 18.2 and 12.8 (one round); head_dim 96
-        // with 32/32 heads at 4k (four per CU) 17.0 against 23.1 (one round);
-        // head_dim 64 with 12/3 heads at 8k 9.5 against 10.6 (one round).
-        const long long units = dense_tiles * 8 + static_cast<long long>(blocks_ub) * W;
-        const long long rounds = res.per_cu >= 4 ? 2 : 1;
-        const long long cap = std::max<long long>(1, units * rounds / 8);
+        // At least a unit of work per wave and at most one round of resident
+        // workgroups (per launch with its merge: head_dim 80 with 32/32 heads
+        // at 2k 10.7 us, 13.8 with a second round), for head_dim above 128 at
+        // most two per CU (16/8 heads at 8k 15.8 us against 16.8 with the
+        // three that fit). Past 128 slots per head the merge and the mean
+        // weights read the split statistics in more than one pass, so there a
+        // wave first gets eight units (head_dim 64 with 9/3 heads at 32k 17.7
+        // us with 128 slots, 19.4 with 512; head_dim 96 with 12/4 heads at 8k
+        // 12.1 against 12.8 with 192). Whole groups of 8 slots: slot s of
+        // every head runs on XCD s % 8, where the heads share the lines of a
+        // token's V words.
+        const int unit = split_unit_tokens(D);
+        const long long units =
+            (static_cast<long long>(dense_ub) + unit - 1) / unit + static_cast<long long>(blocks_ub) * W;
+        const long long cap = D > 128 ? std::min<long long>(resident, 2LL * res.cus) : resident;
+        long long ns = std::min((cap + heads - 1) / heads, std::max<long long>(128, units / 32));
+        ns = std::max<long long>(1, std::min(ns, (units + 3) / 4));
+        if (fewer) ns = (ns + 1) / 2;
+        if (ns >= 8) ns = (ns + 7) / 8 * 8;
         p.nsplit_p = 0;
-        p.nsplit_d = static_cast<int>(std::max<long long>(1, std::min(rounds * per_head, cap)));
+        p.nsplit_d = static_cast<int>(ns);
     }
     p.nsplit = p.nsplit_p + p.nsplit_d;
     p.token_ub = dense_ub + blocks_ub * kgs;
@@ -1435,8 +1520,6 @@ int attn_launch_split(const AttnInputs& real_in, const AttnPlan& plan, void* ws,
     a.nsplit = plan.nsplit;
     a.nsplit_p = plan.nsplit_p;
     a.nsplit_d = plan.nsplit_d;
-    a.wd = 8;
-    a.wp = 1;
     a.dense_delay = plan.dense_delay;
     const int G = in.Hq / in.Hkv;
     const int gp = gp_for(G);
