@@ -508,16 +508,55 @@ struct PrefillArgs {
     int chunk, sink, nbq, rem, q_len, short_path, s, r;
 };
 
-__global__ void prefill_state_kernel(PrefillArgs a) {
+// Token rows that a prefill keeps in f32: rows [row, row + rows) of the prompt
+// to k_dst / v_dst.
+struct PrefillRows {
+    float* k_dst;
+    float* v_dst;
+    int row, rows;
+};
+struct PrefillCopy {
+    const float* k;
+    const float* v;
+    size_t kvs;
+    int vec;  // floats per copy: 4 where the prompt is 16-byte aligned, else 1
+    PrefillRows part[3];
+};
+
+// The f32 rows of a prefill and its bookkeeping in one launch. Workgroup 0
+// writes the ids and the state, which must follow every read of the old block
+// count (its barrier; the quantisers ran before); the others copy.
+__global__ void __launch_bounds__(1024) prefill_rows_kernel(PrefillArgs a, PrefillCopy c) {
+    if (blockIdx.x > 0) {
+        const size_t t0 = (blockIdx.x - 1) * static_cast<size_t>(blockDim.x) + threadIdx.x;
+        const size_t stride = (gridDim.x - 1) * static_cast<size_t>(blockDim.x);
+        for (const PrefillRows& p : c.part) {
+            const float* k = c.k + p.row * c.kvs;
+            const float* v = c.v + p.row * c.kvs;
+            const size_t n = p.rows * c.kvs;  // kvs: a multiple of 16
+            if (c.vec == 4) {
+                for (size_t i = 4 * t0; i < n; i += 4 * stride) {
+                    const float4 x = *reinterpret_cast<const float4*>(k + i), y = *reinterpret_cast<const float4*>(v + i);
+                    *reinterpret_cast<float4*>(p.k_dst + i) = x;
+                    *reinterpret_cast<float4*>(p.v_dst + i) = y;
+                }
+            } else {
+                for (size_t i = t0; i < n; i += stride) {
+                    p.k_dst[i] = k[i];
+                    p.v_dst[i] = v[i];
+                }
+            }
+        }
+        return;
+    }
     int* st = a.st;
     const int used = st[kBlocksUsed];
-    for (int i = threadIdx.x + blockIdx.x * blockDim.x; i < a.nbq * a.chunk; i += blockDim.x * gridDim.x)
+    for (int i = threadIdx.x; i < a.nbq * a.chunk; i += blockDim.x)
         a.pbs_ids[static_cast<size_t>(used) * a.chunk + i] = a.sink + i;
     const int rs = a.sink + a.nbq * a.chunk;
-    for (int t = threadIdx.x + blockIdx.x * blockDim.x; t < a.rem; t += blockDim.x * gridDim.x) a.wr_ids[t] = rs + t;
-    // Every thread has read `used` before thread 0 of block 0 rewrites it.
+    for (int t = threadIdx.x; t < a.rem; t += blockDim.x) a.wr_ids[t] = rs + t;
     __syncthreads();
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (threadIdx.x == 0) {
         if (a.short_path) {
             if (a.s > 0) st[kSCount] = a.s;
             if (a.r > 0) {
@@ -586,13 +625,33 @@ __global__ void __launch_bounds__(256) feedback_kernel(const int* st, const floa
     }
 }
 
-template <typename T>
-int dev_alloc(T** p, size_t n) {
-    void* v = nullptr;
-    TT_HIP_CHECK(hipMalloc(&v, std::max<size_t>(n, 1) * sizeof(T)));
-    *p = static_cast<T*>(v);
-    return TT_OK;
-}
+// Lays buffers out behind one another in one device allocation (an engine's
+// buffers in an allocation each took about 15 us apiece to make and to free).
+// take() registers a buffer, alloc() makes the allocation and sets them all.
+class Arena {
+public:
+    template <typename T>
+    void take(T** p, const size_t n) {
+        parts_.push_back({reinterpret_cast<void**>(p), size_});
+        size_ += (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~static_cast<size_t>(255);
+    }
+    size_t size() const { return size_; }
+    int alloc(char** base) {
+        void* v = nullptr;
+        TT_HIP_CHECK(hipMalloc(&v, size_));
+        *base = static_cast<char*>(v);
+        for (const Part& q : parts_) *q.p = *base + q.off;
+        return TT_OK;
+    }
+
+private:
+    struct Part {
+        void** p;
+        size_t off;
+    };
+    std::vector<Part> parts_;
+    size_t size_ = 0;
+};
 
 }  // namespace
 }  // namespace tt
@@ -609,8 +668,10 @@ struct tt_engine {
     float *HH_scores = nullptr, *WR_K = nullptr, *WR_V = nullptr, *EV_K = nullptr, *EV_V = nullptr, *g = nullptr;
     int64_t *HH_ids = nullptr, *WR_ids = nullptr, *PBS_ids = nullptr;
     int32_t *PBS_KP = nullptr, *PBS_VP = nullptr;
-    void *PBS_KS = nullptr, *PBS_KZ = nullptr, *PBS_VS = nullptr, *PBS_VZ = nullptr;
+    char *PBS_KS = nullptr, *PBS_KZ = nullptr, *PBS_VS = nullptr, *PBS_VZ = nullptr;
     int cap_blocks = 0;
+    char* tiers = nullptr;  // the allocation of everything but the packed store
+    char* pbs = nullptr;    // the allocation of the packed store
     int* st = nullptr;
     unsigned int* ts = nullptr;  // threshold selection state (kThrStateWords)
     // host mirror of the data-independent counters
@@ -625,7 +686,7 @@ struct tt_engine {
     size_t ws_bytes = 0;
     float* mw = nullptr;
     size_t mw_cap = 0;
-    int* host_state = nullptr;  // pinned
+    int host_state[kStateSlots] = {};
     // A step whose mean weights and score feedback are still to run (its
     // partials, logits and row statistics are in ws): tt_engine_step_deferred
     // leaves it for the next engine's finalize launch or a flush.
@@ -637,17 +698,6 @@ struct tt_engine {
 };
 
 namespace {
-
-int engine_free_pbs(tt_engine* e) {
-    (void)hipFree(e->PBS_KP);
-    (void)hipFree(e->PBS_VP);
-    (void)hipFree(e->PBS_KS);
-    (void)hipFree(e->PBS_KZ);
-    (void)hipFree(e->PBS_VS);
-    (void)hipFree(e->PBS_VZ);
-    (void)hipFree(e->PBS_ids);
-    return TT_OK;
-}
 
 int engine_reserve_ws(tt_engine* e, const AttnPlan& p, hipStream_t s);
 
@@ -665,14 +715,21 @@ int engine_reserve_blocks(tt_engine* e, int need, hipStream_t s) {
     const int nc = std::max(need, e->cap_blocks + std::max(64, e->cap_blocks / 2));
     const size_t kvs = e->kvs, ch = e->chunk, msz = e->msz(), W = e->kgs / 16;
     int32_t *kp, *vp;
-    char *ks, *kz, *vs, *vz;
+    char *ks, *kz, *vs, *vz, *pbs;
     int64_t* ids;
-    int rc;
-    if ((rc = dev_alloc(&kp, nc * W * kvs)) || (rc = dev_alloc(&vp, nc * ch * e->Hkv * e->qhd)) ||
-        (rc = dev_alloc(&ks, nc * kvs * msz)) || (rc = dev_alloc(&kz, nc * kvs * msz)) ||
-        (rc = dev_alloc(&vs, nc * ch * e->Hkv * msz)) || (rc = dev_alloc(&vz, nc * ch * e->Hkv * msz)) ||
-        (rc = dev_alloc(&ids, nc * ch)))
-        return rc;
+    Arena arena;
+    arena.take(&kp, nc * W * kvs);
+    arena.take(&vp, nc * ch * e->Hkv * e->qhd);
+    arena.take(&ks, nc * kvs * msz);
+    arena.take(&kz, nc * kvs * msz);
+    arena.take(&vs, nc * ch * e->Hkv * msz);
+    arena.take(&vz, nc * ch * e->Hkv * msz);
+    const size_t zeroed = arena.size();
+    arena.take(&ids, nc * ch);
+    const int rc = arena.alloc(&pbs);
+    if (rc) return rc;
+    // unused blocks are zeros with ids -1
+    TT_HIP_CHECK(hipMemsetAsync(pbs, 0, zeroed, s));
     const size_t ob = e->cap_blocks;
     if (ob > 0) {
         TT_HIP_CHECK(hipMemcpyAsync(kp, e->PBS_KP, ob * W * kvs * 4, hipMemcpyDeviceToDevice, s));
@@ -683,16 +740,11 @@ int engine_reserve_blocks(tt_engine* e, int need, hipStream_t s) {
         TT_HIP_CHECK(hipMemcpyAsync(vz, e->PBS_VZ, ob * ch * e->Hkv * msz, hipMemcpyDeviceToDevice, s));
         TT_HIP_CHECK(hipMemcpyAsync(ids, e->PBS_ids, ob * ch * 8, hipMemcpyDeviceToDevice, s));
         TT_HIP_CHECK(hipStreamSynchronize(s));
-        engine_free_pbs(e);
+        (void)hipFree(e->pbs);
     }
-    TT_HIP_CHECK(hipMemsetAsync(kp + ob * W * kvs, 0, (nc - ob) * W * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(vp + ob * ch * e->Hkv * e->qhd, 0, (nc - ob) * ch * e->Hkv * e->qhd * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(ks + ob * kvs * msz, 0, (nc - ob) * kvs * msz, s));
-    TT_HIP_CHECK(hipMemsetAsync(kz + ob * kvs * msz, 0, (nc - ob) * kvs * msz, s));
-    TT_HIP_CHECK(hipMemsetAsync(vs + ob * ch * e->Hkv * msz, 0, (nc - ob) * ch * e->Hkv * msz, s));
-    TT_HIP_CHECK(hipMemsetAsync(vz + ob * ch * e->Hkv * msz, 0, (nc - ob) * ch * e->Hkv * msz, s));
     hipLaunchKernelGGL(fill_ids_kernel, dim3(64), dim3(256), 0, s, ids, ob * ch, static_cast<size_t>(nc) * ch);
     TT_LAUNCH_CHECK();
+    e->pbs = pbs;
     e->PBS_KP = kp;
     e->PBS_VP = vp;
     e->PBS_KS = ks;
@@ -844,28 +896,29 @@ int tt_engine_create(tt_engine** out, int num_q_heads, int num_kv_heads, int hea
     if (e->max_hh < 1) e->max_hh = 1;
     e->kvs = static_cast<size_t>(num_kv_heads) * head_dim;
     const size_t kvs = e->kvs;
-    if ((rc = dev_alloc(&e->S_K, std::max(1, e->S) * kvs)) || (rc = dev_alloc(&e->S_V, std::max(1, e->S) * kvs)) ||
-        (rc = dev_alloc(&e->RW_K, e->R * kvs)) || (rc = dev_alloc(&e->RW_V, e->R * kvs)) ||
-        (rc = dev_alloc(&e->HH_K, e->max_hh * kvs)) || (rc = dev_alloc(&e->HH_V, e->max_hh * kvs)) ||
-        (rc = dev_alloc(&e->HH_scores, e->max_hh)) || (rc = dev_alloc(&e->HH_ids, e->max_hh)) ||
-        (rc = dev_alloc(&e->WR_K, e->chunk * kvs)) || (rc = dev_alloc(&e->WR_V, e->chunk * kvs)) ||
-        (rc = dev_alloc(&e->WR_ids, e->chunk)) || (rc = dev_alloc(&e->EV_K, kvs)) || (rc = dev_alloc(&e->EV_V, kvs)) ||
-        (rc = dev_alloc(&e->g, e->msl)) || (rc = dev_alloc(&e->st, kStateSlots)) ||
-        (rc = dev_alloc(&e->ts, kThrStateWords))) {
+    Arena arena;
+    arena.take(&e->S_K, std::max(1, e->S) * kvs);
+    arena.take(&e->S_V, std::max(1, e->S) * kvs);
+    arena.take(&e->RW_K, e->R * kvs);
+    arena.take(&e->RW_V, e->R * kvs);
+    arena.take(&e->HH_K, e->max_hh * kvs);
+    arena.take(&e->HH_V, e->max_hh * kvs);
+    arena.take(&e->HH_scores, e->max_hh);
+    arena.take(&e->WR_K, e->chunk * kvs);
+    arena.take(&e->WR_V, e->chunk * kvs);
+    arena.take(&e->ts, kThrStateWords);
+    const size_t zeroed = arena.size();
+    arena.take(&e->HH_ids, e->max_hh);
+    arena.take(&e->WR_ids, e->chunk);
+    arena.take(&e->EV_K, kvs);
+    arena.take(&e->EV_V, kvs);
+    arena.take(&e->g, e->msl);
+    arena.take(&e->st, kStateSlots);
+    if ((rc = arena.alloc(&e->tiers))) {
         tt_engine_destroy(e);
         return rc;
     }
-    TT_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&e->host_state), kStateSlots * sizeof(int)));
-    TT_HIP_CHECK(hipMemsetAsync(e->S_K, 0, std::max(1, e->S) * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->S_V, 0, std::max(1, e->S) * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->RW_K, 0, e->R * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->RW_V, 0, e->R * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->HH_K, 0, e->max_hh * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->HH_V, 0, e->max_hh * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->HH_scores, 0, e->max_hh * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->WR_K, 0, e->chunk * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->WR_V, 0, e->chunk * kvs * 4, s));
-    TT_HIP_CHECK(hipMemsetAsync(e->ts, 0, kThrStateWords * sizeof(unsigned int), s));
+    TT_HIP_CHECK(hipMemsetAsync(e->tiers, 0, zeroed, s));
     const int want_blocks = (e->msl + e->chunk - 1) / e->chunk + 1;
     if ((rc = engine_reserve_blocks(e, want_blocks, s))) {
         tt_engine_destroy(e);
@@ -884,16 +937,10 @@ int tt_engine_destroy(tt_engine* e) {
     if (!e) return TT_OK;
     DeviceGuard dg(e->device);
     (void)hipDeviceSynchronize();
-    float* fb[] = {e->S_K, e->S_V, e->RW_K, e->RW_V, e->HH_K, e->HH_V, e->HH_scores, e->WR_K, e->WR_V, e->EV_K,
-                   e->EV_V, e->g, e->mw};
-    for (float* p : fb) (void)hipFree(p);
-    (void)hipFree(e->HH_ids);
-    (void)hipFree(e->WR_ids);
-    (void)hipFree(e->st);
-    (void)hipFree(e->ts);
+    (void)hipFree(e->tiers);
+    (void)hipFree(e->pbs);
     (void)hipFree(e->ws);
-    engine_free_pbs(e);
-    if (e->host_state) (void)hipHostFree(e->host_state);
+    (void)hipFree(e->mw);
     delete e;
     return TT_OK;
 }
@@ -1160,17 +1207,18 @@ int tt_engine_prefill(tt_engine* e, const float* K_all, const float* V_all, int 
     pa.chunk = e->chunk;
     pa.sink = e->S;
     pa.q_len = q_len;
+    PrefillCopy pc{};
+    pc.k = K_all;
+    pc.v = V_all;
+    pc.kvs = kvs;
+    pc.vec = ((reinterpret_cast<uintptr_t>(K_all) | reinterpret_cast<uintptr_t>(V_all)) & 15) == 0 ? 4 : 1;
     if (q_len <= e->S + e->R) {
         const int sc = std::min(e->S, q_len);
         const int r = q_len - sc;
-        if (sc > 0) {
-            TT_HIP_CHECK(hipMemcpyAsync(e->S_K, K_all, sc * kvs * 4, hipMemcpyDeviceToDevice, s));
-            TT_HIP_CHECK(hipMemcpyAsync(e->S_V, V_all, sc * kvs * 4, hipMemcpyDeviceToDevice, s));
-            e->h_s = sc;
-        }
+        pc.part[0] = {e->S_K, e->S_V, 0, sc};
+        pc.part[1] = {e->RW_K, e->RW_V, sc, r};
+        if (sc > 0) e->h_s = sc;
         if (r > 0) {
-            TT_HIP_CHECK(hipMemcpyAsync(e->RW_K, K_all + sc * kvs, r * kvs * 4, hipMemcpyDeviceToDevice, s));
-            TT_HIP_CHECK(hipMemcpyAsync(e->RW_V, V_all + sc * kvs, r * kvs * 4, hipMemcpyDeviceToDevice, s));
             e->h_rw = r;
             e->h_head = 0;
         }
@@ -1178,17 +1226,14 @@ int tt_engine_prefill(tt_engine* e, const float* K_all, const float* V_all, int 
         pa.s = sc;
         pa.r = r;
     } else {
-        TT_HIP_CHECK(hipMemcpyAsync(e->S_K, K_all, e->S * kvs * 4, hipMemcpyDeviceToDevice, s));
-        TT_HIP_CHECK(hipMemcpyAsync(e->S_V, V_all, e->S * kvs * 4, hipMemcpyDeviceToDevice, s));
         const int rw_start = q_len - e->R;
-        TT_HIP_CHECK(hipMemcpyAsync(e->RW_K, K_all + rw_start * kvs, e->R * kvs * 4, hipMemcpyDeviceToDevice, s));
-        TT_HIP_CHECK(hipMemcpyAsync(e->RW_V, V_all + rw_start * kvs, e->R * kvs * 4, hipMemcpyDeviceToDevice, s));
         const int n_inter = rw_start - e->S;
         const int nbq = n_inter / e->chunk;
         const int rem = n_inter % e->chunk;
         if (nbq > 0) {
             int rc = engine_reserve_blocks(e, e->blocks_ub + nbq + 1, s);
             if (rc) return rc;
+            pa.pbs_ids = e->PBS_ids;
             const float* ksrc = K_all + e->S * kvs;
             const float* vsrc = V_all + e->S * kvs;
             rc = launch_quantize_k(ksrc, reinterpret_cast<uint32_t*>(e->PBS_KP), e->PBS_KS, e->PBS_KZ, nbq, e->Hkv, e->D,
@@ -1198,11 +1243,9 @@ int tt_engine_prefill(tt_engine* e, const float* K_all, const float* V_all, int 
                                    e->st + kBlocksUsed, e->chunk, s);
             if (rc) return rc;
         }
-        if (rem > 0) {
-            const size_t rs = e->S + static_cast<size_t>(nbq) * e->chunk;
-            TT_HIP_CHECK(hipMemcpyAsync(e->WR_K, K_all + rs * kvs, rem * kvs * 4, hipMemcpyDeviceToDevice, s));
-            TT_HIP_CHECK(hipMemcpyAsync(e->WR_V, V_all + rs * kvs, rem * kvs * 4, hipMemcpyDeviceToDevice, s));
-        }
+        pc.part[0] = {e->S_K, e->S_V, 0, e->S};
+        pc.part[1] = {e->RW_K, e->RW_V, rw_start, e->R};
+        pc.part[2] = {e->WR_K, e->WR_V, e->S + nbq * e->chunk, rem};
         pa.short_path = 0;
         pa.nbq = nbq;
         pa.rem = rem;
@@ -1214,11 +1257,11 @@ int tt_engine_prefill(tt_engine* e, const float* K_all, const float* V_all, int 
         e->blocks_ub += nbq;
         e->wr_ub = rem;
     }
-    const int work = std::max(pa.nbq * pa.chunk, pa.rem);
-    // One workgroup: the state update must follow every read of the old
-    // block count, which a block-wide barrier guarantees.
-    (void)work;
-    hipLaunchKernelGGL(prefill_state_kernel, dim3(1), dim3(1024), 0, s, pa);
+    size_t rows = 0;
+    for (const PrefillRows& p : pc.part) rows += p.rows;
+    const size_t wgs = (rows * kvs / pc.vec + 1023) / 1024;
+    hipLaunchKernelGGL(prefill_rows_kernel, dim3(1 + static_cast<unsigned>(std::min<size_t>(wgs, 512))), dim3(1024), 0,
+                       s, pa, pc);
     TT_LAUNCH_CHECK();
     e->h_total = q_len;
     return TT_OK;
@@ -1271,9 +1314,12 @@ int tt_engine_buffer(tt_engine* e, int which, void** p, int64_t* numel, int* es,
     clear_error();
     if (!e || !p || !numel || !es) TT_FAIL(TT_ERR_INVALID_ARGUMENT, "engine or output is NULL.");
     DeviceGuard dg(e->device);
-    int rc = engine_sync_state(e, as_stream(stream));
+    // The tiers of fixed size need no counters from the device; their pending
+    // feedback is enqueued all the same.
+    const bool fixed = (which >= 0 && which <= 10) || which == 18;
+    int rc = fixed ? engine_flush(e, as_stream(stream)) : engine_sync_state(e, as_stream(stream));
     if (rc) return rc;
-    const int64_t kvs = static_cast<int64_t>(e->kvs), nb = e->host_state[kLogicalAlloc], ch = e->chunk;
+    const int64_t kvs = static_cast<int64_t>(e->kvs), nb = fixed ? 0 : e->host_state[kLogicalAlloc], ch = e->chunk;
     const int msz = static_cast<int>(e->msz());
     if (nb > e->cap_blocks) TT_FAIL(TT_ERR_RUNTIME, "packed store smaller than its logical allocation.");
     switch (which) {
