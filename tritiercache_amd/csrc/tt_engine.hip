@@ -52,10 +52,18 @@ __global__ void __launch_bounds__(256) append_row_kernel(const float* __restrict
 // Exact k-th smallest of g[0..n) by an MSB radix select on order-preserving
 // keys, three passes of 11, 11 and 10 bits; any exact selection equals
 // std::nth_element's pick (cache_engine.cpp:126-144). Writes the threshold
-// and last_calc_pos. One workgroup: every thread keeps kThrBatch loads in
-// flight per pass step, and the digit of each pass is found with a parallel
-// prefix sum over the histogram.
-constexpr int kThrBatch = 32;
+// and last_calc_pos. One workgroup for up to kThrOneWg candidates, all of
+// them in registers over the passes; the digit of each pass is found with a
+// parallel prefix sum over the histogram.
+//
+// What it waits for is one read of the scores by one CU and the LDS atomics:
+// scores share few leading digits (after a prefill they are all zero), so a
+// wave adds the lanes that hold its first lane's digit in one atomic. 16k
+// zeros after a prefill: 18 us (50 with an atomic per lane and a read per
+// pass). The spread selection's six launches take about twice the 30 us of
+// 32k candidates here.
+constexpr int kThrPer = 32;
+constexpr int kThrOneWg = 1024 * kThrPer;
 
 __device__ __forceinline__ unsigned int wave_incl_scan(unsigned int x) {
     const int lane = threadIdx.x & 63;
@@ -65,6 +73,24 @@ __device__ __forceinline__ unsigned int wave_incl_scan(unsigned int x) {
         if (lane >= d) x += y;
     }
     return x;
+}
+
+__device__ __forceinline__ unsigned int order_key(const float v) {
+    const unsigned int u = __float_as_uint(v);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// hist[d] += 1 for the lanes with `in` (called by whole waves).
+__device__ __forceinline__ void hist_add(unsigned int* hist, const unsigned int d, const bool in) {
+    const unsigned long long act = __ballot(in);
+    if (act == 0) return;
+    const int lead = __ffsll(static_cast<long long>(act)) - 1;
+    const unsigned int d0 = __builtin_amdgcn_readlane(d, lead);
+    const unsigned long long same = __ballot(in && d == d0);
+    if (static_cast<int>(threadIdx.x & 63) == lead)
+        atomicAdd(&hist[d0], static_cast<unsigned int>(__popcll(same)));
+    else if (in && d != d0)
+        atomicAdd(&hist[d], 1u);
 }
 
 __global__ void __launch_bounds__(1024) threshold_kernel(const float* __restrict__ g, int n, long long k, int* st,
@@ -78,6 +104,12 @@ __global__ void __launch_bounds__(1024) threshold_kernel(const float* __restrict
         s_mask = 0;
         s_k = static_cast<unsigned int>(k);  // k < n < 2^31
     }
+    unsigned int key[kThrPer];
+#pragma unroll
+    for (int j = 0; j < kThrPer; ++j) {
+        const int i = j * 1024 + tid;
+        key[j] = i < n ? order_key(g[i]) : 0u;
+    }
     for (int pass = 0; pass < 3; ++pass) {
         const int bits = pass < 2 ? 11 : 10;
         const int shift = pass == 0 ? 21 : (pass == 1 ? 10 : 0);
@@ -85,18 +117,10 @@ __global__ void __launch_bounds__(1024) threshold_kernel(const float* __restrict
         for (int i = tid; i < 2048; i += 1024) hist[i] = 0;
         __syncthreads();
         const unsigned int prefix = s_prefix, mask = s_mask;
-        for (int base = 0; base < n; base += 1024 * kThrBatch) {
-            unsigned int u[kThrBatch];
 #pragma unroll
-            for (int j = 0; j < kThrBatch; ++j) {
-                const int i = base + j * 1024 + tid;
-                u[j] = i < n ? __float_as_uint(g[i]) : 0u;
-            }
-#pragma unroll
-            for (int j = 0; j < kThrBatch; ++j) {
-                const unsigned int key = (u[j] & 0x80000000u) ? ~u[j] : (u[j] | 0x80000000u);
-                if (base + j * 1024 + tid < n && (key & mask) == prefix) atomicAdd(&hist[(key >> shift) & dm], 1u);
-            }
+        for (int j = 0; j < kThrPer; ++j) {
+            if (j * 1024 >= n) break;
+            hist_add(hist, (key[j] >> shift) & dm, j * 1024 + tid < n && (key[j] & mask) == prefix);
         }
         __syncthreads();
         // Thread t owns bins 2t and 2t + 1; the digit is the bin where the
@@ -136,13 +160,6 @@ __global__ void __launch_bounds__(1024) threshold_kernel(const float* __restrict
 constexpr int kThrHistWgs = 64;   // at most, each 256 threads x kThrHistPer candidates per round
 constexpr int kThrHistPer = 16;
 constexpr int kThrStateWords = 2048 + 4;
-// Candidate counts from which the six launches of the spread selection beat
-// the single-workgroup kernel.
-#ifndef TT_THR_MULTI_MIN
-#define TT_THR_MULTI_MIN 16384
-#endif
-constexpr size_t kThrMultiMin = TT_THR_MULTI_MIN;
-
 __device__ __forceinline__ int thr_bits(int pass) { return pass < 2 ? 11 : 10; }
 __device__ __forceinline__ int thr_shift(int pass) { return pass == 0 ? 21 : (pass == 1 ? 10 : 0); }
 
@@ -157,17 +174,15 @@ __global__ void __launch_bounds__(256) thr_hist_kernel(const float* __restrict__
     const unsigned int prefix = ts[2048], mask = ts[2049];
     const int stride = gridDim.x * 256 * kThrHistPer;
     for (int base = blockIdx.x * 256 * kThrHistPer; base < n; base += stride) {
-        unsigned int u[kThrHistPer];
+        unsigned int key[kThrHistPer];
 #pragma unroll
         for (int j = 0; j < kThrHistPer; ++j) {
             const int i = base + j * 256 + tid;
-            u[j] = i < n ? __float_as_uint(g[i]) : 0u;
+            key[j] = i < n ? order_key(g[i]) : 0u;
         }
 #pragma unroll
-        for (int j = 0; j < kThrHistPer; ++j) {
-            const unsigned int key = (u[j] & 0x80000000u) ? ~u[j] : (u[j] | 0x80000000u);
-            if (base + j * 256 + tid < n && (key & mask) == prefix) atomicAdd(&hist[(key >> shift) & dm], 1u);
-        }
+        for (int j = 0; j < kThrHistPer; ++j)
+            hist_add(hist, (key[j] >> shift) & dm, base + j * 256 + tid < n && (key[j] & mask) == prefix);
     }
     __syncthreads();
     for (int i = tid; i < 2048; i += 256)
@@ -980,7 +995,7 @@ int tt_engine_ingest(tt_engine* e, const float* K_new, const float* V_new, void*
             if (q < 0.0f) q = 0.0f;
             if (q > 1.0f) q = 1.0f;
             const size_t k = static_cast<size_t>(q * static_cast<float>(n - 1));
-            if (n < kThrMultiMin) {
+            if (n <= static_cast<size_t>(kThrOneWg)) {
                 hipLaunchKernelGGL(threshold_kernel, dim3(1), dim3(1024), 0, s, e->g + cs, static_cast<int>(n),
                                    static_cast<long long>(k), e->st, e->h_total);
                 TT_LAUNCH_CHECK();
