@@ -1,5 +1,5 @@
-"""The VALU attention kernel (head dims other than 128, and 64 with an odd number of KV heads) where a wave holds
-several units: more work than one unit per wave of the launch, ragged tails of both kinds, and tiers and queries that
+"""The VALU attention kernel (head dims other than 128, and 64 with an odd number of KV heads) and the merge, where a
+wave holds several units: more work than one unit per wave of the launch, ragged tails of both kinds, and tiers and queries that
 start one element past an aligned address."""
 import numpy as np
 import pytest
@@ -34,6 +34,7 @@ CASES = [
     (5, 5, 16, 1030, 0, 16, False, "none"),       # FP32 tokens only
     (10, 5, 240, 0, 37, 32, False, "tail"),       # packed tokens only
     (12, 3, 48, 17, 1, 16, True, "all"),
+    (2, 1, 128, 40, 3300, 16, False, "holes"),    # one head over the device: more than 256 partial slots to merge
 ]
 
 
