@@ -6,13 +6,13 @@
 // Here each token's K/V bytes are read from HBM once. Logits are kept in
 // log2 units (dot * log2(e) / sqrt(D)) so every exponential is one v_exp_f32.
 //
-//   attn_packed_kernel  head_dim 128: the 2-bit packed blocks on the matrix
+//   attn_packed_kernel  head_dim 128 (64 in pairs): the 2-bit packed blocks on the matrix
 //                       cores (tt_attn_mfma.h), grid (splits, Hkv, head
 //                       chunks), 4 waves; one (max, sum, acc[D]) partial per
 //                       (query head, split).
 //   attn_split_kernel   VALU loop, grid (splits, Hkv, head chunks), 4 waves:
 //                       head_dim other than 128 (and 64 with an odd number of
-//                       KV heads), FP32 tiers and 2-bit tiles, the latter
+//                       KV heads), and short contexts of both: FP32 tiers and 2-bit tiles, the latter
 //                       unpacked in registers with the reference's dequant
 //                       rounding fmaf(q, scale, zero); online softmax over all
 //                       GQA query heads of the KV head.
@@ -24,9 +24,7 @@
 #include "tt_attn.h"
 
 #include <algorithm>
-#include <map>
-#include <mutex>
-#include <tuple>
+#include <atomic>
 
 namespace tt {
 
@@ -87,8 +85,9 @@ struct SplitArgs {
 #include "tt_attn_mfma.h"
 
 // ---------------------------------------------------------------------------
-// The VALU loop (head_dim other than 128, and 64 with an odd number of KV
-// heads). FP32 arithmetic throughout: operands, products and sums.
+// The VALU loop (head_dim other than 128, 64 with an odd number of KV heads,
+// and short contexts of both). FP32 arithmetic throughout: operands, products
+// and sums.
 // ---------------------------------------------------------------------------
 
 // Tokens of one FP32 unit of a wave: half a tile for the head dims whose rows of four tokens per lane would take
@@ -1316,26 +1315,31 @@ const void* split_kernel_ptr(int gp, int fp16) {
 }
 
 // CUs of the device and workgroups of the split launch one CU holds at once
-// (queried once per device and shape, then cached).
+// (queried once per device and instantiation, then read from a table: every
+// call plans, and a plan asks for one or two).
 struct Residency {
     int cus = 256;
     int per_cu = 2;
 };
+constexpr int kResidencyDevices = 64;
 
-Residency split_residency(int D, int G, int fp16, bool pair = false) {
-    static std::mutex mu;
-    static std::map<std::tuple<int, int, int, int, int>, Residency> cache;
+// `valu`: the VALU kernel's, also where the matrix-core kernel serves the head_dim.
+Residency split_residency(int D, int G, int fp16, bool pair = false, bool valu = false) {
+    // cus << 8 | per_cu, 0 where not yet queried (racing queries store the same value)
+    static std::atomic<int> table[kResidencyDevices][2][16][4][2][2];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return Residency{};
     const int gp = gp_for(G);
-    const auto key = std::make_tuple(dev, D, gp, fp16, pair ? 1 : 0);
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = cache.find(key);
-    if (it != cache.end()) return it->second;
+    std::atomic<int>* slot = nullptr;
+    if (dev < kResidencyDevices) {
+        slot = &table[dev][valu ? 1 : 0][D / 16 - 1][gp == 1 ? 0 : gp == 2 ? 1 : gp == 4 ? 2 : 3][fp16 ? 1 : 0][pair ? 1 : 0];
+        const int v = slot->load(std::memory_order_relaxed);
+        if (v) return Residency{v >> 8, v & 255};
+    }
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     const void* fn = nullptr;
-    if (use_packed_kernel(D)) {
+    if (use_packed_kernel(D) && !valu) {
         fn = fp16 ? packed_kernel_ptr<uint16_t>(gp, pair) : packed_kernel_ptr<float>(gp, pair);
     } else {
         // the instantiation the launch runs (channels per lane = head_dim / 16)
@@ -1363,9 +1367,8 @@ Residency split_residency(int D, int G, int fp16, bool pair = false) {
         (void)hipGetLastError();
         per_cu = 2;
     }
-    const Residency r{cus, per_cu};
-    cache[key] = r;
-    return r;
+    if (slot) slot->store(cus << 8 | per_cu, std::memory_order_relaxed);
+    return Residency{cus, per_cu};
 }
 
 }  // namespace
@@ -1385,7 +1388,35 @@ int attn_check_shapes(int Hq, int Hkv, int D, int kgs) {
 
 namespace {
 AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                        int meta_fp16, bool pair, bool fewer);
+                        int meta_fp16, bool pair, bool fewer, bool valu);
+}  // namespace
+
+namespace {
+// Units (16-token tiles of either kind) per KV head up to which the VALU kernel
+// serves the head dims of the matrix-core kernel too. At short contexts a
+// launch is one chain of latencies, and the VALU kernel's is shorter: no
+// lay-out in LDS, no coefficients, a unit per wave. Its arithmetic grows with
+// units x query heads x channels, so the line lies at a share of the units
+// that a resident round of its waves holds one of, below the point where the
+// matrix cores win with blocks of 32 tokens. Partials per launch, VALU against
+// matrix cores, at units per wave:
+//   one head per group of 128: 32/32 heads at 2k (0.8) 7.2 against 8.8 us, at
+//     4k (1.6) 9.9 against 11.3, at 8k (3.2) 17.4 against 15.0;
+//   two: 16/8 at 4k (0.5) 6.6 against 7.4, at 8k (1.0) 9.1 against 7.9;
+//   four: 32/8 at 1k (0.2) 5.7 against 6.3, at 2.5k (0.4) 7.2 against 7.2, at
+//     4k (0.7) 8.3 against 7.5;
+//   more: 28/4 at 1k (0.2) 7.4 against 6.2;
+//   head_dim 64: 32/32 at 2k (0.6) 5.7 against 7.1, 16/16 at 8k (1.2) 8.4
+//     against 8.1; 32/8 at 1k (0.2) 4.6 against 6.3, at 6k (0.7) 7.1 against
+//     7.5; 14/2 at 2k (0.08) 5.9 against 6.3, at 8k (0.3) 8.1 against 6.6.
+long long short_units(int Hq, int Hkv, int D, int meta_fp16) {
+    const int G = Hq / Hkv, gp = gp_for(G);
+    const int eighths = D == 64 ? (gp <= 4 ? 8 : 1) : gp == 1 ? 14 : gp == 2 ? 8 : gp == 4 ? 3 : 0;
+    const long long heads = static_cast<long long>(Hkv) * ((G + gp - 1) / gp);
+    const Residency res = split_residency(D, G, meta_fp16, false, true);
+    return 4LL * res.cus * res.per_cu * eighths / (8 * heads);
+}
+bool use_matrix_cores(int D, int Hkv) { return use_packed_kernel(D) || (D == 64 && Hkv % 2 == 0); }
 }  // namespace
 
 // Head_dim 64 with an even number of KV heads runs as half as many heads of
@@ -1396,27 +1427,41 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
 // head (zeros in the other half), which leaves their logits exact.
 AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16,
                    bool fewer) {
-    if (D == 64 && Hkv % 2 == 0) {
-        AttnPlan p = attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv / 2, kMfD, kgs, need_logits, meta_fp16, true, fewer);
+    const bool pair = D == 64 && Hkv % 2 == 0;
+    const long long units = (static_cast<long long>(dense_ub) + 15) / 16 + static_cast<long long>(blocks_ub) * (kgs / 16);
+    const bool valu = !use_matrix_cores(D, Hkv) || units <= short_units(Hq, Hkv, D, meta_fp16);
+    if (pair && !valu) {
+        AttnPlan p = attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv / 2, kMfD, kgs, need_logits, meta_fp16, true, fewer, false);
         p.pair64 = true;
         return p;
     }
-    return attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv, D, kgs, need_logits, meta_fp16, false, fewer);
+    return attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv, D, kgs, need_logits, meta_fp16, false, fewer, valu);
+}
+
+// The plan of the most units within the bounds that the VALU kernel takes from
+// the matrix cores (its partials can be larger than those at the bounds).
+AttnPlan attn_plan_short(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
+                         int meta_fp16) {
+    const long long units = use_matrix_cores(D, Hkv) ? short_units(Hq, Hkv, D, meta_fp16) : 0;
+    const int W = kgs / 16;
+    const int blocks = static_cast<int>(std::min<long long>(blocks_ub, units / W));
+    const int dense = static_cast<int>(std::min<long long>(dense_ub, 16 * (units - static_cast<long long>(blocks) * W)));
+    return attn_plan(dense, blocks, Hq, Hkv, D, kgs, need_logits, meta_fp16);
 }
 
 namespace {
 AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                        int meta_fp16, bool pair, bool fewer) {
+                        int meta_fp16, bool pair, bool fewer, bool valu) {
     AttnPlan p;
     const int W = kgs / 16;
     const int G = Hq / Hkv;
     const int chunks = (G + gp_for(G) - 1) / gp_for(G);
     const long long heads = static_cast<long long>(Hkv) * chunks;
-    const Residency res = split_residency(D, G, meta_fp16, pair);
+    const Residency res = split_residency(D, G, meta_fp16, pair, valu);
     const long long resident = static_cast<long long>(res.cus) * res.per_cu;
     const long long per_head = std::max<long long>(1, (resident + heads - 1) / heads);
     const long long dense_tiles = (dense_ub + 15) / 16;
-    if (use_packed_kernel(D)) {
+    if (!valu) {
         // One resident round of workgroups per head, at least ~4 units of work
         // each so the partials stay small (a 32-token pair of packed tiles is
         // one unit, a 16-token FP32 tile kDenseTileCost), shared between
@@ -1559,12 +1604,11 @@ int attn_launch_split(const AttnInputs& real_in, const AttnPlan& plan, void* ws,
     const int G = in.Hq / in.Hkv;
     const int gp = gp_for(G);
     const int chunks = (G + gp - 1) / gp;
-    if (use_packed_kernel(in.D)) {
-        if (plan.nsplit_p <= 0) TT_FAIL(TT_ERR_RUNTIME, "attention plan does not match head_dim");
+    if (plan.nsplit_p > 0) {
+        if (!use_packed_kernel(in.D)) TT_FAIL(TT_ERR_RUNTIME, "attention plan does not match head_dim");
         return launch_packed(a, in.Hkv, chunks, gp, in.meta_fp16, plan.pair64, stream);
     }
     const dim3 grid(plan.nsplit, in.Hkv, chunks);
-    if (plan.nsplit_p != 0) TT_FAIL(TT_ERR_RUNTIME, "attention plan does not match head_dim");
     switch (in.D / 16) {
     case 1: return launch_split_g<1>(a, grid, gp, in.meta_fp16, stream);
     case 2: return launch_split_g<2>(a, grid, gp, in.meta_fp16, stream);

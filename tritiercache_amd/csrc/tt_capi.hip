@@ -87,7 +87,7 @@ int check_common(int dense_count, int num_blocks, int Hq, int Hkv, int D, int kg
     return TT_OK;
 }
 
-// Validates the stateless attention arguments and fills the kernel inputs and plan.
+// Validates the stateless attention arguments and fills the kernel inputs and plan (`plan` null: validation only).
 int prepare(const float* Q, const float* dK, const float* dV, int dense_count, const int32_t* KP, const void* KS,
             const void* KZ, const int32_t* VP, const void* VS, const void* VZ, const int64_t* ids, int num_blocks,
             int Hq, int Hkv, int D, int kgs, int meta_fp16, bool want_mw, AttnInputs* in, AttnPlan* plan,
@@ -99,6 +99,7 @@ int prepare(const float* Q, const float* dK, const float* dV, int dense_count, c
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "Argument 'dense_K'/'dense_V' pointer address is NULL.");
     if (num_blocks > 0 && (!KP || !KS || !KZ || !VP || !VS || !VZ || !ids))
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "PBS arguments must be non-NULL when num_blocks > 0.");
+    if (!plan) return TT_OK;
     *plan = attn_plan(dense_count, num_blocks, Hq, Hkv, D, kgs, want_mw, meta_fp16, fewer);
     if (want_mw && !logits_fit(Hq, plan->ld))
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "num_q_heads x tokens exceeds the 4 GiB logits buffer of the mean weights.");
@@ -167,11 +168,9 @@ int check_batch(const tt_decode_seq* seqs, int num_seqs, int Hq, int Hkv, int D,
         const long long tub = static_cast<long long>(q.dense_count) + static_cast<long long>(q.num_blocks) * kgs;
         if (q.mean_attn_weights && !logits_fit(Hq, (tub + 3) & ~3LL))
             TT_FAIL(TT_ERR_INVALID_ARGUMENT, "num_q_heads x tokens exceeds the 4 GiB logits buffer of the mean weights.");
-        AttnInputs in;
-        AttnPlan plan;
         rc = prepare(q.Q, q.dense_K, q.dense_V, q.dense_count, q.PBS_K_Packed, q.PBS_K_Scales, q.PBS_K_Zeroes,
                      q.PBS_V_Packed, q.PBS_V_Scales, q.PBS_V_Zeroes, q.PBS_token_ids, q.num_blocks, Hq, Hkv, D, kgs, 0,
-                     false, &in, &plan);
+                     false, nullptr, nullptr);
         if (rc) return rc;
         if (!q.attn_output) TT_FAIL(TT_ERR_INVALID_ARGUMENT, "Argument 'attn_output' pointer address is NULL.");
     }

@@ -768,8 +768,11 @@ int engine_reserve_blocks(tt_engine* e, int need, hipStream_t s) {
     e->PBS_VZ = vz;
     e->PBS_ids = ids;
     e->cap_blocks = nc;
-    // Attention workspace follows the capacity.
-    return engine_reserve_ws(e, attn_plan(e->S + e->max_hh + e->R, nc, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16), s);
+    // Attention workspace follows the capacity, for every context up to it.
+    const int dense_ub = e->S + e->max_hh + e->R;
+    const int rw = engine_reserve_ws(e, attn_plan(dense_ub, nc, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16), s);
+    if (rw) return rw;
+    return engine_reserve_ws(e, attn_plan_short(dense_ub, nc, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16), s);
 }
 
 // Grows the attention workspace and the mean-weight buffer to what plan `p`
