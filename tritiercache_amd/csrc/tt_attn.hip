@@ -69,6 +69,33 @@ __device__ __forceinline__ void load_f32(const float* __restrict__ p, float (&x)
     }
 }
 
+// A wave-uniform value as a scalar. Counts that come from the engine's device
+// state or from the kernel arguments would otherwise be read with one vector
+// load whose address is selected, a round trip before a workgroup knows its
+// share of the work. (With the tier pointers below: partials of 32/8 heads at
+// 32k 15.0 -> 14.2 us, at 4k 7.5 -> 7.3, head_dim 64 at 32k 11.7 -> 11.3; an
+// engine step of four layers at 4k 69.0 -> 66.4.)
+__device__ __forceinline__ int scalar(const int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// The FP32 tiers' addresses as values in scalar registers: a per-lane choice
+// between them is then a select. (Left to the compiler it becomes a load of the
+// chosen pointer from the kernel arguments, a round trip before each tile's
+// own loads.)
+struct TierPtrs {
+    uint64_t k0, k1, k2, v0, v1, v2;
+};
+__device__ __forceinline__ TierPtrs tier_ptrs(const AttnInputs& in) {
+    auto u = [](const float* p) { return reinterpret_cast<uint64_t>(p); };
+    TierPtrs t{u(in.k0), u(in.k1), u(in.k2), u(in.v0), u(in.v1), u(in.v2)};
+    asm("" : "+s"(t.k0), "+s"(t.k1), "+s"(t.k2), "+s"(t.v0), "+s"(t.v1), "+s"(t.v2));
+    return t;
+}
+// The address of global memory that such a value holds (the type says global, or the loads become flat ones).
+__device__ __forceinline__ const float* global_f32(const uint64_t a) {
+    typedef const __attribute__((address_space(1))) float* gptr;
+    return (const float*)reinterpret_cast<gptr>(a);
+}
+
 struct SplitArgs {
     AttnInputs in;
     float scale2;  // log2(e) / sqrt(head_dim): logits are kept in log2 units
@@ -230,13 +257,12 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
     }
 
     int n0 = in.n0, n1 = in.n1, n2 = in.n2, head = in.ring_head, nb = in.num_blocks;
-    auto uniform = [](const int x) { return __builtin_amdgcn_readfirstlane(x); };
     if (in.state) {
-        n0 = uniform(in.state[kSCount]);
-        n1 = uniform(in.state[kHhCount]);
-        n2 = uniform(in.state[kRwCount]);
-        head = uniform(in.state[kRwHead]);
-        nb = uniform(in.state[kBlocksUsed]);
+        n0 = scalar(in.state[kSCount]);
+        n1 = scalar(in.state[kHhCount]);
+        n2 = scalar(in.state[kRwCount]);
+        head = scalar(in.state[kRwHead]);
+        nb = scalar(in.state[kBlocksUsed]);
     }
     const int Nd = n0 + n1 + n2;
     const int W = in.kgs >> 4;
@@ -299,13 +325,14 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
         }
     };
 
+    const TierPtrs tier = tier_ptrs(in);
 #pragma unroll 1
     for (int k = d_begin; k < d_end; ++k) {
         // ---- FP32 unit: logical rows 4 NTD k ... ----
         const int tok0 = 4 * NTD * k;
         float kx[NTD][CPL], vx[NTD][CPL];
         size_t off[NTD];
-        const float* vb[NTD];
+        uint64_t vb[NTD];
 #pragma unroll
         for (int i = 0; i < NTD; ++i) {
             const int r = min(tok0 + tg + 4 * i, Nd - 1);  // rows past the tiers are masked below
@@ -314,11 +341,11 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
             ring = ring >= in.ring_size ? ring - in.ring_size : ring;
             const int idx = in0 ? r : (in1 ? r - n0 : ring);
             off[i] = (static_cast<size_t>(idx) * Hkv + kvh) * D + cp * CPL;
-            vb[i] = in0 ? in.v0 : (in1 ? in.v1 : in.v2);
-            load_slice<CPL>((in0 ? in.k0 : (in1 ? in.k1 : in.k2)) + off[i], kx[i]);
+            vb[i] = in0 ? tier.v0 : (in1 ? tier.v1 : tier.v2);
+            load_slice<CPL>(global_f32(in0 ? tier.k0 : (in1 ? tier.k1 : tier.k2)) + off[i], kx[i]);
         }
 #pragma unroll
-        for (int i = 0; i < NTD; ++i) load_slice<CPL>(vb[i] + off[i], vx[i]);
+        for (int i = 0; i < NTD; ++i) load_slice<CPL>(global_f32(vb[i]) + off[i], vx[i]);
         float s[NTD][GP];
 #pragma unroll
         for (int i = 0; i < NTD; ++i)

@@ -337,7 +337,7 @@ __device__ __forceinline__ void load_q_lds(const AttnInputs& in, const int kvh, 
     }
 }
 
-// Tier pointers and counts of the FP32 tokens (device counters for the engine).
+// Counts of the FP32 tokens (device counters for the engine).
 struct DenseView {
     int n0, n1, n2, head, Nd;
 };
@@ -345,10 +345,10 @@ struct DenseView {
 __device__ __forceinline__ DenseView dense_view(const AttnInputs& in) {
     DenseView v{in.n0, in.n1, in.n2, in.ring_head, 0};
     if (in.state) {
-        v.n0 = in.state[kSCount];
-        v.n1 = in.state[kHhCount];
-        v.n2 = in.state[kRwCount];
-        v.head = in.state[kRwHead];
+        v.n0 = scalar(in.state[kSCount]);
+        v.n1 = scalar(in.state[kHhCount]);
+        v.n2 = scalar(in.state[kRwCount]);
+        v.head = scalar(in.state[kRwHead]);
     }
     v.Nd = v.n0 + v.n1 + v.n2;
     return v;
@@ -364,6 +364,9 @@ struct DenseTile {
     float4 v[4][2];
 };
 
+// LEAN: the tier pointers from the kernel arguments, for the one kernel (paired
+// eight-head groups) whose other branch would spill a register with all six in
+// scalars.
 // K and V rows of token `r0` (clamped to the last tier row; rows past the
 // tiers are masked later) in the logical FP32 order sinks -> heavy hitters ->
 // recent ring.
@@ -371,32 +374,38 @@ struct DenseRow {
     const float* k;
     const float* v;
 };
+template <bool LEAN>
 __device__ __forceinline__ DenseRow dense_row(const AttnInputs& in, const DenseView& dv, const int kvh, const int r0) {
     const int r = r0 < dv.Nd ? r0 : dv.Nd - 1;
     const bool in0 = r < dv.n0, in1 = r < dv.n0 + dv.n1;
     int ring = dv.head + (r - dv.n0 - dv.n1);
     ring = ring >= in.ring_size ? ring - in.ring_size : ring;
     const int idx = in0 ? r : (in1 ? r - dv.n0 : ring);
-    const float* kb = in0 ? in.k0 : (in1 ? in.k1 : in.k2);
-    const float* vb = in0 ? in.v0 : (in1 ? in.v1 : in.v2);
     const size_t off = (static_cast<size_t>(idx) * in.Hkv + kvh) * kMfD;
-    return DenseRow{kb + off, vb + off};
+    if constexpr (LEAN) {
+        const float* kb = in0 ? in.k0 : (in1 ? in.k1 : in.k2);
+        const float* vb = in0 ? in.v0 : (in1 ? in.v1 : in.v2);
+        return DenseRow{kb + off, vb + off};
+    }
+    const TierPtrs t = tier_ptrs(in);
+    return DenseRow{global_f32(in0 ? t.k0 : (in1 ? t.k1 : t.k2)) + off, global_f32(in0 ? t.v0 : (in1 ? t.v1 : t.v2)) + off};
 }
 
 // Issues the loads of tile k.
+template <bool LEAN>
 __device__ __forceinline__ void dense_load(const AttnInputs& in, const DenseView& dv, const int kvh, const int k,
                                            DenseTile& t) {
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, n = lane & 15;
     const int tok0 = 16 * k;
     {
-        const float* kb = dense_row(in, dv, kvh, tok0 + n).k + 32 * g;
+        const float* kb = dense_row<LEAN>(in, dv, kvh, tok0 + n).k + 32 * g;
 #pragma unroll
         for (int i = 0; i < 8; ++i) t.k[i] = *reinterpret_cast<const float4*>(kb + 4 * i);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float* vb = dense_row(in, dv, kvh, tok0 + 4 * g + j).v + 8 * n;
+        const float* vb = dense_row<LEAN>(in, dv, kvh, tok0 + 4 * g + j).v + 8 * n;
         t.v[j][0] = *reinterpret_cast<const float4*>(vb);
         t.v[j][1] = *reinterpret_cast<const float4*>(vb + 4);
     }
@@ -409,6 +418,7 @@ struct DenseTileV {
     float kx[4][8], vx[4][8];
 };
 
+template <bool LEAN>
 __device__ __forceinline__ void dense_load(const AttnInputs& in, const DenseView& dv, const int kvh, const int k,
                                            DenseTileV& t) {
     const int lane = threadIdx.x & 63;
@@ -416,7 +426,7 @@ __device__ __forceinline__ void dense_load(const AttnInputs& in, const DenseView
     const int tok0 = 16 * k + 4 * tg;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const DenseRow r = dense_row(in, dv, kvh, tok0 + i);
+        const DenseRow r = dense_row<LEAN>(in, dv, kvh, tok0 + i);
         load_f32<8>(r.k + 8 * cp, t.kx[i]);
         load_f32<8>(r.v + 8 * cp, t.vx[i]);
     }
@@ -514,7 +524,7 @@ __device__ __forceinline__ void dense_share_valu(const SplitArgs& a, const Dense
 #pragma unroll 1
     for (int k = kb; k < d1; k += 4) {
         DenseTileV t;
-        dense_load(in, dv, kvh, k, t);
+        dense_load<false>(in, dv, kvh, k, t);
         consume(t, k);
     }
     // The four token groups share m: sum them, then the partial into LDS.
@@ -567,7 +577,7 @@ __device__ __forceinline__ float4 mfma4x4f32(const float a, const float b, const
 // 2^16 factor), so most tiles skip the rescale. Leaves one (max, sum,
 // acc[128]) partial per head in `dl` ([GP][2 + 128] per wave) and writes
 // the logits.
-template <int GP>
+template <int GP, bool LEAN>
 __device__ __forceinline__ void dense_share(const SplitArgs& a, const DenseView& dv, const int d0, const int d1,
                                             const int kvh, const int g0, const int gc, const int wave,
                                             const float* q_l, const DenseTile& t0, float* dl) {
@@ -649,7 +659,7 @@ __device__ __forceinline__ void dense_share(const SplitArgs& a, const DenseView&
 #pragma unroll 1
     for (int k = kb; k < d1; k += 4) {
         DenseTile t;
-        dense_load(in, dv, kvh, k, t);
+        dense_load<LEAN>(in, dv, kvh, k, t);
         consume(t, k);
     }
     // The head's sum over its four lane groups, then the partial in LDS:
@@ -698,14 +708,15 @@ __device__ __forceinline__ void dense_body(const SplitArgs& a, const int dsplit,
     }
     if constexpr (GP <= 2) {
         DenseTileV dt;
-        if (d0 + wave < d1) dense_load(in, dv, kvh, d0 + wave, dt);
+        if (d0 + wave < d1) dense_load<false>(in, dv, kvh, d0 + wave, dt);
         __syncthreads();
         dense_share_valu<GP>(a, dv, d0, d1, kvh, g0, gc, wave, q_l, dt, dl);
     } else {
+        constexpr bool kLean = PAIR && GP == 8;
         DenseTile dt;
-        if (d0 + wave < d1) dense_load(in, dv, kvh, d0 + wave, dt);
+        if (d0 + wave < d1) dense_load<kLean>(in, dv, kvh, d0 + wave, dt);
         __syncthreads();
-        dense_share<GP>(a, dv, d0, d1, kvh, g0, gc, wave, q_l, dt, dl);
+        dense_share<GP, kLean>(a, dv, d0, d1, kvh, g0, gc, wave, q_l, dt, dl);
     }
     __syncthreads();
     const int split = a.nsplit_p + dsplit;
@@ -753,6 +764,7 @@ template <int GP, typename MetaT, bool PAIR = false>
 __device__ __forceinline__ void packed_body(const SplitArgs& a, const int split, const int kvh, const int chunk,
                                             char* lds) {
     static_assert(GP >= 1 && GP <= 8, "at most 8 query heads per workgroup");
+    constexpr bool kLeanSel = PAIR && GP == 8;  // no register to spare (see below and dense_row)
     constexpr int NP = GP >= 4 ? GP / 4 : 1;  // coefficient passes (4 heads x 16 chunks each)
     using L = MfLds<GP>;
     const AttnInputs& in = a.in;
@@ -778,6 +790,12 @@ __device__ __forceinline__ void packed_body(const SplitArgs& a, const int split,
         n1 = in.state[kHhCount];
         n2 = in.state[kRwCount];
         nb = in.state[kBlocksUsed];
+        if constexpr (!kLeanSel) {
+            n0 = scalar(n0);
+            n1 = scalar(n1);
+            n2 = scalar(n2);
+            nb = scalar(nb);
+        }
     }
     const int Nd = n0 + n1 + n2;
     const int W = in.kgs >> 4;
@@ -932,7 +950,6 @@ __device__ __forceinline__ void packed_body(const SplitArgs& a, const int split,
     // byte selectors of the V transpose (paired eight-head groups recompute
     // them in the lay-out from an opaque copy of the thread id: held over the
     // loop they would push that kernel past 168 VGPRs)
-    constexpr bool kLeanSel = PAIR && GP == 8;
     const uint32_t qsel1_c = (lane & 1) ? 0x03070105u : 0x06020400u;
     const uint32_t qsel2_c = (lane & 2) ? 0x03020706u : 0x05040100u;
 
