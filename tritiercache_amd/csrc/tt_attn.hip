@@ -90,11 +90,19 @@ __device__ __forceinline__ TierPtrs tier_ptrs(const AttnInputs& in) {
     asm("" : "+s"(t.k0), "+s"(t.k1), "+s"(t.k2), "+s"(t.v0), "+s"(t.v1), "+s"(t.v2));
     return t;
 }
-// The address of global memory that such a value holds (the type says global, or the loads become flat ones).
-__device__ __forceinline__ const float* global_f32(const uint64_t a) {
-    typedef const __attribute__((address_space(1))) float* gptr;
-    return (const float*)reinterpret_cast<gptr>(a);
+// A pointer into global memory whose origin does not tell (an integer, or read
+// from memory): without the address space in its type the accesses become flat
+// ones, which LDS waits include.
+template <typename T>
+__device__ __forceinline__ T* global_ptr(const uint64_t a) {
+    typedef __attribute__((address_space(1))) T* gptr;
+    return (T*)reinterpret_cast<gptr>(a);
 }
+template <typename T>
+__device__ __forceinline__ T* global_ptr(T* p) {
+    return global_ptr<T>(reinterpret_cast<uint64_t>(p));
+}
+__device__ __forceinline__ const float* global_f32(const uint64_t a) { return global_ptr<const float>(a); }
 
 struct SplitArgs {
     AttnInputs in;
@@ -1150,17 +1158,17 @@ attn_batched_kernel(const BatchArgs b) {
     }
     const tt_decode_seq& d = b.seqs[i];
     SplitArgs a;
-    a.in.Q = d.Q;
-    a.in.k0 = d.dense_K;
-    a.in.v0 = d.dense_V;
+    a.in.Q = global_ptr(d.Q);
+    a.in.k0 = global_ptr(d.dense_K);
+    a.in.v0 = global_ptr(d.dense_V);
     a.in.n0 = d.dense_count;
-    a.in.kp = d.PBS_K_Packed;
-    a.in.ks = d.PBS_K_Scales;
-    a.in.kz = d.PBS_K_Zeroes;
-    a.in.vp = d.PBS_V_Packed;
-    a.in.vs = d.PBS_V_Scales;
-    a.in.vz = d.PBS_V_Zeroes;
-    a.in.ids = d.PBS_token_ids;
+    a.in.kp = global_ptr(d.PBS_K_Packed);
+    a.in.ks = global_ptr(d.PBS_K_Scales);
+    a.in.kz = global_ptr(d.PBS_K_Zeroes);
+    a.in.vp = global_ptr(d.PBS_V_Packed);
+    a.in.vs = global_ptr(d.PBS_V_Scales);
+    a.in.vz = global_ptr(d.PBS_V_Zeroes);
+    a.in.ids = global_ptr(d.PBS_token_ids);
     a.in.num_blocks = d.num_blocks;
     a.in.Hq = b.Hq;
     a.in.Hkv = b.Hkv;
@@ -1206,14 +1214,14 @@ __device__ __forceinline__ FinArgs fin_batch_args(const FinBatchArgs& b, const i
     a.D = kMfD;
     a.Hq = b.Hq;
     a.pair_g = 0;
-    a.out = d.attn_output;
+    a.out = global_ptr(d.attn_output);
     a.rowstat = b.rowstat + static_cast<size_t>(i) * 2 * b.Hq;
     a.logits = d.mean_attn_weights ? b.logits + static_cast<size_t>(b.tok_base[i]) * b.Hq : nullptr;
     a.ld = b.tok_base[i + 1] - b.tok_base[i];
     a.n_static = d.dense_count + d.num_blocks * b.kgs;
     a.state = nullptr;
     a.kgs = b.kgs;
-    a.mw = d.mean_attn_weights;
+    a.mw = global_ptr(d.mean_attn_weights);
     a.head_w = nullptr;
     a.head_w_ld = 0;
     a.fb = Feedback{};
