@@ -673,7 +673,7 @@ __device__ __forceinline__ void fin_merge_head(const FinArgs& a, const int h, co
 #pragma unroll
         for (int u = 0; u < kMergeU; ++u) {
             v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (u * groups < nj)  // splits past the last re-read it and are given no weight
+            if (u * groups < nj)  // splits past the last re-read it and are not added
                 v[u] = *reinterpret_cast<const float4*>(base + static_cast<size_t>(j0 + min(g + u * groups, nj - 1)) * a.D);
         }
         // the whole block's statistics in every wave, so that no wave waits for another
@@ -692,19 +692,26 @@ __device__ __forceinline__ void fin_merge_head(const FinArgs& a, const int h, co
         if (j0 > 0) {
             A.x *= al; A.y *= al; A.z *= al; A.w *= al;
         }
-        auto add = [&](const int j, const float4 x) {
-            const float f = (g < groups && j < nj) ? own[j] : 0.0f;
+        auto add = [&](const float f, const float4 x) {
             A.x = __builtin_fmaf(f, x.x, A.x);
             A.y = __builtin_fmaf(f, x.y, A.y);
             A.z = __builtin_fmaf(f, x.z, A.z);
             A.w = __builtin_fmaf(f, x.w, A.w);
         };
+        // (a re-read split is replaced by zeros rather than given a zero factor alone: its sums may be infinite;
+        // threads past the last whole group add what nothing reads)
 #pragma unroll
-        for (int u = 0; u < kMergeU; ++u)
-            if (u * groups < nj) add(g + u * groups, v[u]);
+        for (int u = 0; u < kMergeU; ++u) {
+            if (u * groups < nj) {
+                const int j = g + u * groups;
+                const bool in = j < nj;
+                add(own[min(j, nj - 1)], make_float4(in ? v[u].x : 0.0f, in ? v[u].y : 0.0f, in ? v[u].z : 0.0f,
+                                                     in ? v[u].w : 0.0f));
+            }
+        }
         // splits beyond kMergeU per group in this block of 256 (groups < 16 only)
         for (int j = g + kMergeU * groups; g < groups && j < nj; j += groups)
-            add(j, *reinterpret_cast<const float4*>(base + static_cast<size_t>(j0 + j) * a.D));
+            add(own[j], *reinterpret_cast<const float4*>(base + static_cast<size_t>(j0 + j) * a.D));
         wave_lds_sync();
     }
     // Sum over the groups: within a wave across its rows where a group's
