@@ -41,3 +41,17 @@ def check(oracle, case, seed):
 @pytest.mark.parametrize("case", MERGE, ids=str)
 def test_merge_adds_no_slot_twice(oracle, case):
     check(oracle, case, seed=2100 + MERGE.index(case))
+
+# ragged ends of the VALU kernel's FP32 units
+UNIT = [
+    (9, 3, 64, 16 * 63 + 5, 0),   # 64 units, 16 slots (as many as the merge has groups)
+    (2, 2, 80, 1, 0),
+    (8, 8, 256, 8 * 31 + 1, 2),   # units of 8 tokens
+    (4, 2, 128, 37, 3),           # short contexts of head_dim 128
+    (5, 5, 16, 17, 0),
+]
+
+
+@pytest.mark.parametrize("case", UNIT, ids=str)
+def test_fp32_unit_weighs_no_row_twice(oracle, case):
+    check(oracle, case, seed=2200 + UNIT.index(case))

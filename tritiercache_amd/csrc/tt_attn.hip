@@ -367,6 +367,14 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
             }
         if (a.logits) put_logits(s, tok0, Nd);
         softmax(s);
+        // Rows past the tiers repeat the last one, whose V may be infinite: a
+        // zero weight alone would make a NaN of it.
+        if (tok0 + 4 * NTD > Nd) {
+#pragma unroll
+            for (int i = 0; i < NTD; ++i)
+#pragma unroll
+                for (int j = 0; j < CPL; ++j) vx[i][j] = (tok0 + tg + 4 * i < Nd) ? vx[i][j] : 0.0f;
+        }
 #pragma unroll
         for (int i = 0; i < NTD; ++i)
 #pragma unroll
