@@ -5,6 +5,10 @@ registers can make the compiler spill to scratch, which slows the kernel by
 a large factor while every parity test still passes. This test compiles
 tt_attn.hip for gfx950 with the resource remarks and checks, per kernel
 instantiation, the VGPR count, the scratch size and the occupancy.
+
+The VALU kernel takes short contexts of head_dim 128 and 64 up to a line that
+was measured at a number of waves per SIMD; the same compilation checks that
+its instantiations still have them.
 """
 import os
 import re
@@ -58,3 +62,15 @@ def test_no_spills_three_waves(resources, kernel, gp):
         assert res["ScratchSize"] <= LIMITS[gp], (name, res)
         assert res["VGPRs"] <= 168, (name, res)
         assert res["Occupancy"] >= 3, (name, res)
+
+
+# (channels per lane, heads per group): waves per SIMD at which the line between the kernels was measured
+SPLIT_WAVES = {(8, 1): 5, (8, 2): 4, (8, 4): 3, (4, 1): 7, (4, 2): 5, (4, 4): 4, (4, 8): 3}
+
+
+@pytest.mark.parametrize("cpl,gp", SPLIT_WAVES)
+def test_short_context_kernel_keeps_its_waves(resources, cpl, gp):
+    found = {k: v for k, v in resources.items() if f"attn_split_kernelILi{cpl}ELi{gp}E" in k}
+    assert len(found) == 2, sorted(found)  # fp32 and fp16 metadata
+    for name, res in found.items():
+        assert res["ScratchSize"] == 0 and res["Occupancy"] >= SPLIT_WAVES[cpl, gp], (name, res)

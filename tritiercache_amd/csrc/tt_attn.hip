@@ -239,7 +239,9 @@ __device__ __forceinline__ float rows_sum4(const float (&v)[4]) {
 // tile at head_dim 256 with two heads, 350 at head_dim 80 with one), the next
 // unit, the merge. What it responds to is the length of that chain: 32-bit
 // shares of the work (64-bit divides took about 2 us), loads as wide as the
-// row allows from scalar bases, and registers for three to six waves per SIMD.
+// row allows from scalar bases, and registers for as many waves per SIMD as the
+// heads of a group leave (seven at head_dim 64 with one head, three at 128 with
+// four, two at 128 and one at 256 with eight).
 // Partials per launch: head_dim 256 with 16/8 heads at 8k 18.7 -> 11.6 us,
 // head_dim 80 with 32/32 heads at 2k 10.3 -> 6.2, head_dim 96 with 32/32
 // heads at 4k 15.2 -> 9.1, head_dim 64 with 9/3 heads at 8k 9.4 -> 6.4.
@@ -339,6 +341,9 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
         // ---- FP32 unit: logical rows 4 NTD k ... ----
         const int tok0 = 4 * NTD * k;
         float kx[NTD][CPL], vx[NTD][CPL];
+        // (V's addresses up to head_dim 128 at once, from byte offsets, which takes up to ten registers less than a base
+        // and an offset each; above, where two waves per SIMD are planned for, the latter is 0.1 to 0.3 us faster.)
+        constexpr bool kBytes = D <= 128;
         size_t off[NTD];
         uint64_t vb[NTD];
 #pragma unroll
@@ -349,11 +354,18 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
             ring = ring >= in.ring_size ? ring - in.ring_size : ring;
             const int idx = in0 ? r : (in1 ? r - n0 : ring);
             off[i] = (static_cast<size_t>(idx) * Hkv + kvh) * D + cp * CPL;
+            const uint64_t kb = in0 ? tier.k0 : (in1 ? tier.k1 : tier.k2);
             vb[i] = in0 ? tier.v0 : (in1 ? tier.v1 : tier.v2);
-            load_slice<CPL>(global_f32(in0 ? tier.k0 : (in1 ? tier.k1 : tier.k2)) + off[i], kx[i]);
+            if constexpr (kBytes) {
+                const uint64_t bytes = sizeof(float) * off[i];
+                vb[i] += bytes;
+                load_slice<CPL>(global_f32(kb + bytes), kx[i]);
+            } else {
+                load_slice<CPL>(global_f32(kb) + off[i], kx[i]);
+            }
         }
 #pragma unroll
-        for (int i = 0; i < NTD; ++i) load_slice<CPL>(global_f32(vb[i]) + off[i], vx[i]);
+        for (int i = 0; i < NTD; ++i) load_slice<CPL>(global_f32(vb[i]) + (kBytes ? 0 : off[i]), vx[i]);
         float s[NTD][GP];
 #pragma unroll
         for (int i = 0; i < NTD; ++i)
@@ -524,8 +536,11 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
     }
 }
 
+// (Four heads of 128 channels are held to three waves per SIMD: 168 registers,
+// no spills. With two, 32/8 heads at 2k take 7.0 us per launch instead of 5.9.)
 template <int CPL, int GP, typename MetaT>
-__global__ void __launch_bounds__(256) attn_split_kernel(SplitArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((CPL == 8 && GP == 4) ? 3 : 1)))
+attn_split_kernel(SplitArgs a) {
     __shared__ __align__(16) char lds[SplitLds<CPL, GP>::BYTES];
     split_body<CPL, GP, MetaT>(a, static_cast<int>(blockIdx.x), lds);
 }
@@ -1446,25 +1461,29 @@ namespace {
 // serves the head dims of the matrix-core kernel too. At short contexts a
 // launch is one chain of latencies, and the VALU kernel's is shorter: no
 // lay-out in LDS, no coefficients, a unit per wave. Its arithmetic grows with
-// units x query heads x channels, so the line lies at a share of the units
-// that a resident round of its waves holds one of, below the point where the
-// matrix cores win with blocks of 32 tokens. Partials per launch, VALU against
-// matrix cores, at units per wave:
-//   one head per group of 128: 32/32 heads at 2k (0.8) 7.2 against 8.8 us, at
-//     4k (1.6) 9.9 against 11.3, at 8k (3.2) 17.4 against 15.0;
-//   two: 16/8 at 4k (0.5) 6.6 against 7.4, at 8k (1.0) 9.1 against 7.9;
-//   four: 32/8 at 1k (0.2) 5.7 against 6.3, at 2.5k (0.4) 7.2 against 7.2, at
-//     4k (0.7) 8.3 against 7.5;
-//   more: 28/4 at 1k (0.2) 7.4 against 6.2;
-//   head_dim 64: 32/32 at 2k (0.6) 5.7 against 7.1, 16/16 at 8k (1.2) 8.4
-//     against 8.1; 32/8 at 1k (0.2) 4.6 against 6.3, at 6k (0.7) 7.1 against
-//     7.5; 14/2 at 2k (0.08) 5.9 against 6.3, at 8k (0.3) 8.1 against 6.6.
+// units x query heads x channels, so the line is a number of units x heads per
+// CU for each group size and head dim, below the point where the matrix cores
+// win with blocks of 32 tokens. It was measured with the waves per SIMD that
+// the resource test of this kernel asks for (another register count moves the
+// times, not the line). Partials per launch, VALU against matrix cores, at
+// units x heads per CU:
+//   one head per group of 128 (line at 35): 32/32 heads at 2k (18) 6.7 against
+//     8.9 us, at 4k (32) 9.9 against 11.9, at 5k (39) 10.2 against 10.8, at
+//     6k (47) 12.5 against 12.0;
+//   two (16): 16/8 heads at 4k (8) 5.7 against 7.9, at 8k (16) 7.6 against 7.9;
+//   four (4.5): 32/8 heads at 580 (1.1) 5.5 against 5.9, at 2k (4.0) 5.9 against
+//     7.0, at 2.3k (4.5) 7.0 against 7.0, at 3k (5.9) 7.3 against 7.2;
+//   more: 28/4 heads at 1k (1) 7.4 against 6.2;
+//   head_dim 64: one (28): 64/64 heads at 1.5k (24) 6.9 against 8.2, at 2.6k
+//     (41) 9.8 against 9.6; two (20): 32/16 heads at 5k (20) 7.2 against 8.5;
+//     four (16): 32/8 heads at 6k (12) 6.9 against 7.5, at 8k (16) 8.0 against
+//     8.0; more (1.5): 14/2 heads at 3k (1.5) 6.2 against 6.4.
 long long short_units(int Hq, int Hkv, int D, int meta_fp16) {
     const int G = Hq / Hkv, gp = gp_for(G);
-    const int eighths = D == 64 ? (gp <= 4 ? 8 : 1) : gp == 1 ? 14 : gp == 2 ? 8 : gp == 4 ? 3 : 0;
+    const int halves = D == 64 ? (gp == 1 ? 56 : gp == 2 ? 40 : gp == 4 ? 32 : 3)
+                               : (gp == 1 ? 70 : gp == 2 ? 32 : gp == 4 ? 9 : 0);
     const long long heads = static_cast<long long>(Hkv) * ((G + gp - 1) / gp);
-    const Residency res = split_residency(D, G, meta_fp16, false, true);
-    return 4LL * res.cus * res.per_cu * eighths / (8 * heads);
+    return static_cast<long long>(split_residency(D, G, meta_fp16, false, true).cus) * halves / (2 * heads);
 }
 bool use_matrix_cores(int D, int Hkv) { return use_packed_kernel(D) || (D == 64 && Hkv % 2 == 0); }
 }  // namespace
