@@ -75,9 +75,11 @@ struct AttnPlan {
 // `fewer`: half of the VALU kernel's partial slots, for a caller whose workspace is fixed.
 AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16,
                    bool fewer = false);
-// The largest plan within these bounds among the short contexts, whose kernel and split differ.
-AttnPlan attn_plan_short(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                         int meta_fp16);
+// Workspace bytes that hold the plan of every context of at most these dense
+// tokens and blocks (a shorter one can run on another kernel, or under another
+// layout, with more slots).
+size_t attn_workspace_bytes(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
+                            int meta_fp16);
 
 // Enqueues split + merge (+ mean weights / feedback / per-head weights).
 // mean_w: [token count] or null; head_w: [Hq, head_w_ld] or null.

@@ -1507,18 +1507,54 @@ AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs,
     return attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv, D, kgs, need_logits, meta_fp16, false, fewer, valu);
 }
 
-// The plan of the most units within the bounds that the VALU kernel takes from
-// the matrix cores (its partials can be larger than those at the bounds).
-AttnPlan attn_plan_short(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                         int meta_fp16) {
-    const long long units = use_matrix_cores(D, Hkv) ? short_units(Hq, Hkv, D, meta_fp16) : 0;
-    const int W = kgs / 16;
-    const int blocks = static_cast<int>(std::min<long long>(blocks_ub, units / W));
-    const int dense = static_cast<int>(std::min<long long>(dense_ub, 16 * (units - static_cast<long long>(blocks) * W)));
-    return attn_plan(dense, blocks, Hq, Hkv, D, kgs, need_logits, meta_fp16);
+namespace {
+constexpr long long kDenseTileCost = 4;  // a 16-token FP32 tile in units of a packed pair (~3.7x the bytes)
+
+// Work units of the matrix-core kernel: packed pairs of 32 tokens and, priced in them, FP32 tiles.
+long long matrix_units(const int dense_ub, const int blocks_ub, const int kgs) {
+    return (static_cast<long long>(blocks_ub) * (kgs / 16) + 1) / 2 +
+           (static_cast<long long>(dense_ub) + 15) / 16 * kDenseTileCost;
+}
+// Units of the VALU kernel, and its slots per head.
+long long valu_units(const int dense_ub, const int blocks_ub, const int D, const int kgs) {
+    const int unit = split_unit_tokens(D);
+    return (static_cast<long long>(dense_ub) + unit - 1) / unit + static_cast<long long>(blocks_ub) * (kgs / 16);
+}
+int valu_slots(const long long units, const long long heads, const int D, const Residency& res, const bool fewer) {
+    // At least a unit of work per wave and at most one round of resident
+    // workgroups (per launch with its merge: head_dim 80 with 32/32 heads
+    // at 2k 10.7 us, 13.8 with a second round), for head_dim above 128 at
+    // most two per CU (16/8 heads at 8k 15.8 us against 16.8 with the
+    // three that fit). Past 128 slots per head the merge and the mean
+    // weights read the split statistics in more than one pass, so there a
+    // wave first gets eight units (head_dim 64 with 9/3 heads at 32k 17.7
+    // us with 128 slots, 19.4 with 512; head_dim 96 with 12/4 heads at 8k
+    // 12.1 against 12.8 with 192). Whole groups of 8 slots: slot s of
+    // every head runs on XCD s % 8, where the heads share the lines of a
+    // token's V words.
+    const long long resident = static_cast<long long>(res.cus) * res.per_cu;
+    const long long cap = D > 128 ? std::min<long long>(resident, 2LL * res.cus) : resident;
+    long long ns = std::min((cap + heads - 1) / heads, std::max<long long>(128, units / 32));
+    ns = std::max<long long>(1, std::min(ns, (units + 3) / 4));
+    if (fewer) ns = (ns + 1) / 2;
+    if (ns >= 8) ns = (ns + 7) / 8 * 8;
+    return static_cast<int>(ns);
 }
 
-namespace {
+// Workspace offsets and size of a plan whose slots, logits row stride and want of logits are set.
+void plan_layout(AttnPlan& p, const int Hq, const int D) {
+    size_t off = 0;
+    p.off_ml = off;
+    off = align256(off + sizeof(float) * 2 * static_cast<size_t>(Hq) * p.nsplit);
+    p.off_acc = off;
+    off = align256(off + sizeof(float) * static_cast<size_t>(Hq) * p.nsplit * D);
+    p.off_rowstat = off;
+    off = align256(off + sizeof(float) * 2 * static_cast<size_t>(Hq));
+    p.off_logits = off;
+    if (p.logits) off = align256(off + sizeof(float) * static_cast<size_t>(Hq) * std::max(p.ld, 4));
+    p.bytes = off;
+}
+
 AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
                         int meta_fp16, bool pair, bool fewer, bool valu) {
     AttnPlan p;
@@ -1543,7 +1579,6 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
         // sends slot groups of every head to the XCDs round-robin, so a round
         // of `cus / heads` slots lands one workgroup on every CU, and every CU
         // then runs the same mix of packed and FP32 work.
-        constexpr long long kDenseTileCost = 4;  // ~3.7x the bytes of a pair
         const long long pairs = (static_cast<long long>(blocks_ub) * W + 1) / 2;
         const long long dense_units = dense_tiles * kDenseTileCost;
         const long long units = pairs + dense_units;
@@ -1609,45 +1644,51 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
             p.dense_delay = static_cast<int>(std::min<long long>(550, burst / 19000));
         }
     } else {
-        // At least a unit of work per wave and at most one round of resident
-        // workgroups (per launch with its merge: head_dim 80 with 32/32 heads
-        // at 2k 10.7 us, 13.8 with a second round), for head_dim above 128 at
-        // most two per CU (16/8 heads at 8k 15.8 us against 16.8 with the
-        // three that fit). Past 128 slots per head the merge and the mean
-        // weights read the split statistics in more than one pass, so there a
-        // wave first gets eight units (head_dim 64 with 9/3 heads at 32k 17.7
-        // us with 128 slots, 19.4 with 512; head_dim 96 with 12/4 heads at 8k
-        // 12.1 against 12.8 with 192). Whole groups of 8 slots: slot s of
-        // every head runs on XCD s % 8, where the heads share the lines of a
-        // token's V words.
-        const int unit = split_unit_tokens(D);
-        const long long units =
-            (static_cast<long long>(dense_ub) + unit - 1) / unit + static_cast<long long>(blocks_ub) * W;
-        const long long cap = D > 128 ? std::min<long long>(resident, 2LL * res.cus) : resident;
-        long long ns = std::min((cap + heads - 1) / heads, std::max<long long>(128, units / 32));
-        ns = std::max<long long>(1, std::min(ns, (units + 3) / 4));
-        if (fewer) ns = (ns + 1) / 2;
-        if (ns >= 8) ns = (ns + 7) / 8 * 8;
         p.nsplit_p = 0;
-        p.nsplit_d = static_cast<int>(ns);
+        p.nsplit_d = valu_slots(valu_units(dense_ub, blocks_ub, D, kgs), heads, D, res, fewer);
     }
     p.nsplit = p.nsplit_p + p.nsplit_d;
     p.token_ub = dense_ub + blocks_ub * kgs;
     p.ld = (p.token_ub + 3) & ~3;
     p.logits = need_logits;
-    size_t off = 0;
-    p.off_ml = off;
-    off = align256(off + sizeof(float) * 2 * static_cast<size_t>(Hq) * p.nsplit);
-    p.off_acc = off;
-    off = align256(off + sizeof(float) * static_cast<size_t>(Hq) * p.nsplit * D);
-    p.off_rowstat = off;
-    off = align256(off + sizeof(float) * 2 * static_cast<size_t>(Hq));
-    p.off_logits = off;
-    if (need_logits) off = align256(off + sizeof(float) * static_cast<size_t>(Hq) * std::max(p.ld, 4));
-    p.bytes = off;
+    plan_layout(p, Hq, D);
     return p;
 }
+
+// Matrix-core slots per head that no context of at most `units` work units
+// exceeds (the plan's own number can fall as a context grows): the share that
+// its two layouts start from, and one more where the FP32 tiers take it all.
+long long matrix_slots(const long long units, const long long heads, const Residency& res) {
+    const long long resident = static_cast<long long>(res.cus) * res.per_cu;
+    const long long share = std::max<long long>(1, std::min((resident + heads - 1) / heads, units / 4));
+    return (share >= 8 ? (share + 7) / 8 * 8 : share) + 1;
+}
 }  // namespace
+
+size_t attn_workspace_bytes(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
+                            int meta_fp16) {
+    const int G = Hq / Hkv;
+    AttnPlan p;
+    p.token_ub = dense_ub + blocks_ub * kgs;
+    p.ld = (p.token_ub + 3) & ~3;
+    p.logits = need_logits;
+    size_t bytes = 0;
+    long long units = valu_units(dense_ub, blocks_ub, D, kgs);
+    if (use_matrix_cores(D, Hkv)) {
+        units = std::min(units, short_units(Hq, Hkv, D, meta_fp16));
+        const bool pair = D == 64;
+        const int g = pair ? 2 * G : G, hkv = pair ? Hkv / 2 : Hkv;
+        const long long heads = static_cast<long long>(hkv) * ((g + gp_for(g) - 1) / gp_for(g));
+        p.nsplit = static_cast<int>(matrix_slots(matrix_units(dense_ub, blocks_ub, kgs), heads,
+                                                 split_residency(kMfD, g, meta_fp16, pair)));
+        plan_layout(p, Hq, kMfD);
+        bytes = p.bytes;
+    }
+    const long long heads = static_cast<long long>(Hkv) * ((G + gp_for(G) - 1) / gp_for(G));
+    p.nsplit = valu_slots(units, heads, D, split_residency(D, G, meta_fp16, false, true), false);
+    plan_layout(p, Hq, D);
+    return std::max(bytes, p.bytes);
+}
 
 int attn_launch_split(const AttnInputs& real_in, const AttnPlan& plan, void* ws, hipStream_t stream) {
     if (plan.logits && !logits_fit(real_in.Hq, plan.ld))

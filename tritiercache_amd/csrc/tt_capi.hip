@@ -141,7 +141,8 @@ int fused_impl(const float* Q, const float* dK, const float* dV, int dense_count
     if (phase == kFinalize && mw && !logits)
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "mean_attn_weights requested but the partials were planned without them.");
     if (own_ws) {
-        rc = get_workspace(plan.bytes, &ws);
+        // for every shorter context too: a call captured after a longer one allocates nothing
+        rc = get_workspace(attn_workspace_bytes(dense_count, num_blocks, Hq, Hkv, D, kgs, logits, meta_fp16), &ws);
         if (rc) return rc;
     } else if (!ws || ws_bytes < plan.bytes) {
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "workspace is NULL or smaller than tt_fused_attention_workspace_bytes().");
@@ -179,14 +180,18 @@ int check_batch(const tt_decode_seq* seqs, int num_seqs, int Hq, int Hkv, int D,
 
 // Workspace of a batch: the largest launch (chunks of kMaxBatchSeqs sequences
 // run one after another on the stream and share it); other head dims run the
-// sequences one at a time.
-size_t batch_bytes(const tt_decode_seq* seqs, int num_seqs, int Hq, int Hkv, int D, int kgs, int meta_fp16) {
+// sequences one at a time (`shorter`: with room for every shorter context of
+// each, as the size query of a single call has).
+size_t batch_bytes(const tt_decode_seq* seqs, int num_seqs, int Hq, int Hkv, int D, int kgs, int meta_fp16,
+                   bool shorter) {
     size_t b = 0;
     if (!use_packed_kernel(D)) {
-        for (int i = 0; i < num_seqs; ++i)
-            b = std::max(b, attn_plan(seqs[i].dense_count, seqs[i].num_blocks, Hq, Hkv, D, kgs,
-                                      seqs[i].mean_attn_weights != nullptr, meta_fp16)
-                                .bytes);
+        for (int i = 0; i < num_seqs; ++i) {
+            const tt_decode_seq& q = seqs[i];
+            const bool logits = q.mean_attn_weights != nullptr;
+            b = std::max(b, shorter ? attn_workspace_bytes(q.dense_count, q.num_blocks, Hq, Hkv, D, kgs, logits, meta_fp16)
+                                    : attn_plan(q.dense_count, q.num_blocks, Hq, Hkv, D, kgs, logits, meta_fp16).bytes);
+        }
         return b;
     }
     for (int c0 = 0; c0 < num_seqs; c0 += kMaxBatchSeqs)
@@ -321,17 +326,16 @@ size_t tt_fused_attention_workspace_bytes(int dense_count, int num_blocks, int n
                                           int head_dim, int k_group_size, int want_mean_weights) {
     clear_error();
     if (check_common(dense_count, num_blocks, num_q_heads, num_kv_heads, head_dim, k_group_size) != TT_OK) return 0;
-    // The largest plan over both metadata types (their split counts can differ).
-    size_t b = 0;
-    for (int f = 0; f < 2; ++f) {
-        const AttnPlan p = attn_plan(dense_count, num_blocks, num_q_heads, num_kv_heads, head_dim, k_group_size,
-                                     want_mean_weights != 0, f);
-        if (want_mean_weights && !logits_fit(num_q_heads, p.ld)) {
-            set_error("num_q_heads x tokens exceeds the 4 GiB logits buffer of the mean weights.");
-            return 0;
-        }
-        b = std::max(b, p.bytes);
+    const long long tokens = static_cast<long long>(dense_count) + static_cast<long long>(num_blocks) * k_group_size;
+    if (want_mean_weights && !logits_fit(num_q_heads, (tokens + 3) & ~3LL)) {
+        set_error("num_q_heads x tokens exceeds the 4 GiB logits buffer of the mean weights.");
+        return 0;
     }
+    // The larger over both metadata types (their split counts can differ).
+    size_t b = 0;
+    for (int f = 0; f < 2; ++f)
+        b = std::max(b, attn_workspace_bytes(dense_count, num_blocks, num_q_heads, num_kv_heads, head_dim, k_group_size,
+                                             want_mean_weights != 0, f));
     return b;
 }
 
@@ -417,8 +421,8 @@ size_t tt_batched_decode_workspace_bytes(const tt_decode_seq* seqs, int num_seqs
     if (check_batch(seqs, num_seqs, num_q_heads, num_kv_heads, head_dim, k_group_size) != TT_OK) return 0;
     if (num_seqs == 0) return 256;
     // The largest plan over both metadata types (their split counts can differ).
-    return std::max(batch_bytes(seqs, num_seqs, num_q_heads, num_kv_heads, head_dim, k_group_size, 0),
-                    batch_bytes(seqs, num_seqs, num_q_heads, num_kv_heads, head_dim, k_group_size, 1));
+    return std::max(batch_bytes(seqs, num_seqs, num_q_heads, num_kv_heads, head_dim, k_group_size, 0, true),
+                    batch_bytes(seqs, num_seqs, num_q_heads, num_kv_heads, head_dim, k_group_size, 1, true));
 }
 
 int tt_fused_attention_decode_batched(const tt_decode_seq* seqs, const tt_decode_seq* seqs_device, int num_seqs,
@@ -429,7 +433,7 @@ int tt_fused_attention_decode_batched(const tt_decode_seq* seqs, const tt_decode
     int rc = check_batch(seqs, num_seqs, Hq, Hkv, D, kgs);
     if (rc) return rc;
     if (num_seqs == 0) return TT_OK;
-    if (!workspace || workspace_bytes < batch_bytes(seqs, num_seqs, Hq, Hkv, D, kgs, meta_fp16))
+    if (!workspace || workspace_bytes < batch_bytes(seqs, num_seqs, Hq, Hkv, D, kgs, meta_fp16, false))
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "workspace is NULL or smaller than tt_batched_decode_workspace_bytes().");
     const hipStream_t s = as_stream(stream);
     if (!use_packed_kernel(D)) {

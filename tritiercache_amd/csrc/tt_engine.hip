@@ -714,7 +714,7 @@ struct tt_engine {
 
 namespace {
 
-int engine_reserve_ws(tt_engine* e, const AttnPlan& p, hipStream_t s);
+int engine_reserve_ws(tt_engine* e, size_t bytes, int tokens, hipStream_t s);
 
 constexpr int kLogicalSlack = 64;
 
@@ -770,24 +770,22 @@ int engine_reserve_blocks(tt_engine* e, int need, hipStream_t s) {
     e->cap_blocks = nc;
     // Attention workspace follows the capacity, for every context up to it.
     const int dense_ub = e->S + e->max_hh + e->R;
-    const int rw = engine_reserve_ws(e, attn_plan(dense_ub, nc, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16), s);
-    if (rw) return rw;
-    return engine_reserve_ws(e, attn_plan_short(dense_ub, nc, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16), s);
+    return engine_reserve_ws(e, attn_workspace_bytes(dense_ub, nc, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16),
+                             dense_ub + nc * e->kgs, s);
 }
 
-// Grows the attention workspace and the mean-weight buffer to what plan `p`
-// needs (plans for smaller bounds are not always smaller).
-int engine_reserve_ws(tt_engine* e, const AttnPlan& p, hipStream_t s) {
-    if (p.bytes > e->ws_bytes) {
+// Grows the attention workspace to `bytes` and the mean-weight buffer to `tokens`.
+int engine_reserve_ws(tt_engine* e, size_t bytes, int tokens, hipStream_t s) {
+    if (bytes > e->ws_bytes) {
         if (e->ws) {
             TT_HIP_CHECK(hipStreamSynchronize(s));
             (void)hipFree(e->ws);
         }
         e->ws = nullptr;
-        TT_HIP_CHECK(hipMalloc(&e->ws, p.bytes));
-        e->ws_bytes = p.bytes;
+        TT_HIP_CHECK(hipMalloc(&e->ws, bytes));
+        e->ws_bytes = bytes;
     }
-    const size_t tok = static_cast<size_t>(p.token_ub) + 16;
+    const size_t tok = static_cast<size_t>(tokens) + 16;
     if (tok > e->mw_cap) {
         if (e->mw) {
             TT_HIP_CHECK(hipStreamSynchronize(s));
@@ -1076,7 +1074,7 @@ static int engine_attend(tt_engine* e, const float* Q, float* out, float* head_w
     if (rc) return rc;
     const int dense_ub = e->h_s + e->h_routed + e->h_rw;
     const AttnPlan p = attn_plan(dense_ub, e->blocks_ub, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16);
-    rc = engine_reserve_ws(e, p, s);
+    rc = engine_reserve_ws(e, p.bytes, p.token_ub, s);
     if (rc) return rc;
     AttnInputs in = engine_inputs(e, Q);
     Feedback fb = engine_feedback_args(e);
@@ -1109,7 +1107,7 @@ int tt_engine_step_deferred(tt_engine* e, const float* Q, const float* K_new, co
     if (rc) return rc;
     const int dense_ub = e->h_s + e->h_routed + e->h_rw;
     const AttnPlan p = attn_plan(dense_ub, e->blocks_ub, e->Hq, e->Hkv, e->D, e->kgs, true, e->fp16);
-    rc = engine_reserve_ws(e, p, s);
+    rc = engine_reserve_ws(e, p.bytes, p.token_ub, s);
     if (rc) return rc;
     const AttnInputs in = engine_inputs(e, Q);
     rc = attn_launch_split(in, p, e->ws, s);
