@@ -133,9 +133,12 @@ TT_API int tt_fused_attention_decode_ws(const float* Q, const float* dense_K, co
  * forbid hipMalloc): the computation of tt_fused_attention_decode, with its
  * scratch in a static device array of the library (32 MiB, held by every GPU
  * the library runs on until the process ends) instead of an allocated
- * workspace. Calls no hipMalloc/hipFree. A call whose workspace would exceed
- * 32 MiB (tt_fused_attention_workspace_bytes) fails with
- * TT_ERR_INVALID_ARGUMENT and enqueues nothing. All calls on one GPU share that
+ * workspace. Calls no hipMalloc/hipFree. A call whose plan needs more than 32
+ * MiB runs with fewer partial slots where those are what does not fit (head
+ * sizes of the VALU kernel; the result differs in the order of its sums only);
+ * otherwise it fails with TT_ERR_INVALID_ARGUMENT and enqueues nothing. A call
+ * for which tt_fused_attention_workspace_bytes returns at most 32 MiB always
+ * runs. All calls on one GPU share that
  * GPU's array: calls that overlap on one GPU (other streams, other host
  * threads) race on it. */
 TT_API int tt_fused_attention_decode_noalloc(const float* Q, const float* dense_K, const float* dense_V,

@@ -1,5 +1,6 @@
 """The workspace size a caller asks for its longest context holds for every shorter one: contexts on both sides of the
-line between the kernels, in one workspace, with and without mean weights."""
+line between the kernels, in one workspace, with and without mean weights. And the static scratch takes every call
+that it can hold."""
 import ctypes
 
 import numpy as np
@@ -52,3 +53,23 @@ def test_shorter_contexts_in_the_longest_ones_workspace(oracle, Hq, Hkv, D, nd, 
             ro, rmw = oracle.fused_attention_decode(Q.cpu().numpy(), *args[1:11], blocks, *args[12:])
             err = attention_errors(host(out), ro, *((host(mw), rmw) if weights else ()))
             assert attention_ok(err), (blocks, err)
+
+
+@pytest.mark.parametrize("D", [16, 80, 112, 144, 192, 208, 224, 256])
+def test_noalloc_takes_what_fits_with_a_slot_per_head(D):
+    """The largest context whose logits, row statistics and one partial slot per head fit the static scratch is taken
+    by the _noalloc call, and one more block is not (no launch: the output's NULL pointer is refused after the
+    scratch's check)."""
+    from tritiercache_amd import _lib
+
+    L = _lib.load()
+    p, up = 0x10000, lambda x: (x + 255) & ~255  # noqa: E731
+    for Hq, Hkv in ((8, 8), (24, 3), (12, 3), (20, 5), (40, 10), (80, 10), (56, 14), (160, 20), (160, 40)):
+        def taken(nb):
+            rc = L.tt_fused_attention_decode_noalloc(p, p, p, 0, p, p, p, p, p, p, p, nb, Hq, Hkv, D, None, p, 16, 0, None)
+            assert rc == 1
+            return "attn_output" in _lib.last_error()
+
+        fixed = up(8 * Hq) + up(4 * Hq * D) + up(8 * Hq)
+        nb = ((32 << 20) - fixed) // (4 * Hq * 16)
+        assert taken(nb) and taken(nb - 30) and not taken(nb + 1), (Hq, Hkv, D, nb, _lib.last_error())

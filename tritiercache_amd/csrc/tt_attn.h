@@ -72,9 +72,9 @@ struct AttnPlan {
 };
 
 // Plans the split-K launch for an upper bound of dense tokens / blocks.
-// `fewer`: half of the VALU kernel's partial slots, for a caller whose workspace is fixed.
+// `halvings`: how often the VALU kernel's partial slots are halved, for a caller whose workspace is fixed.
 AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16,
-                   bool fewer = false);
+                   int halvings = 0);
 // Workspace bytes that hold the plan of every context of at most these dense
 // tokens and blocks (a shorter one can run on another kernel, or under another
 // layout, with more slots).

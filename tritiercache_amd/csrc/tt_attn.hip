@@ -1453,7 +1453,7 @@ int attn_check_shapes(int Hq, int Hkv, int D, int kgs) {
 
 namespace {
 AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                        int meta_fp16, bool pair, bool fewer, bool valu);
+                        int meta_fp16, bool pair, int halvings, bool valu);
 }  // namespace
 
 namespace {
@@ -1495,16 +1495,16 @@ bool use_matrix_cores(int D, int Hkv) { return use_packed_kernel(D) || (D == 64 
 // query heads of both form one group whose queries fill the half of their own
 // head (zeros in the other half), which leaves their logits exact.
 AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16,
-                   bool fewer) {
+                   int halvings) {
     const bool pair = D == 64 && Hkv % 2 == 0;
     const long long units = (static_cast<long long>(dense_ub) + 15) / 16 + static_cast<long long>(blocks_ub) * (kgs / 16);
     const bool valu = !use_matrix_cores(D, Hkv) || units <= short_units(Hq, Hkv, D, meta_fp16);
     if (pair && !valu) {
-        AttnPlan p = attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv / 2, kMfD, kgs, need_logits, meta_fp16, true, fewer, false);
+        AttnPlan p = attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv / 2, kMfD, kgs, need_logits, meta_fp16, true, halvings, false);
         p.pair64 = true;
         return p;
     }
-    return attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv, D, kgs, need_logits, meta_fp16, false, fewer, valu);
+    return attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv, D, kgs, need_logits, meta_fp16, false, halvings, valu);
 }
 
 namespace {
@@ -1520,7 +1520,7 @@ long long valu_units(const int dense_ub, const int blocks_ub, const int D, const
     const int unit = split_unit_tokens(D);
     return (static_cast<long long>(dense_ub) + unit - 1) / unit + static_cast<long long>(blocks_ub) * (kgs / 16);
 }
-int valu_slots(const long long units, const long long heads, const int D, const Residency& res, const bool fewer) {
+int valu_slots(const long long units, const long long heads, const int D, const Residency& res, const int halvings) {
     // At least a unit of work per wave and at most one round of resident
     // workgroups (per launch with its merge: head_dim 80 with 32/32 heads
     // at 2k 10.7 us, 13.8 with a second round), for head_dim above 128 at
@@ -1536,7 +1536,7 @@ int valu_slots(const long long units, const long long heads, const int D, const 
     const long long cap = D > 128 ? std::min<long long>(resident, 2LL * res.cus) : resident;
     long long ns = std::min((cap + heads - 1) / heads, std::max<long long>(128, units / 32));
     ns = std::max<long long>(1, std::min(ns, (units + 3) / 4));
-    if (fewer) ns = (ns + 1) / 2;
+    ns = (ns + (1LL << halvings) - 1) >> halvings;
     if (ns >= 8) ns = (ns + 7) / 8 * 8;
     return static_cast<int>(ns);
 }
@@ -1556,7 +1556,7 @@ void plan_layout(AttnPlan& p, const int Hq, const int D) {
 }
 
 AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits,
-                        int meta_fp16, bool pair, bool fewer, bool valu) {
+                        int meta_fp16, bool pair, int halvings, bool valu) {
     AttnPlan p;
     const int W = kgs / 16;
     const int G = Hq / Hkv;
@@ -1645,7 +1645,7 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
         }
     } else {
         p.nsplit_p = 0;
-        p.nsplit_d = valu_slots(valu_units(dense_ub, blocks_ub, D, kgs), heads, D, res, fewer);
+        p.nsplit_d = valu_slots(valu_units(dense_ub, blocks_ub, D, kgs), heads, D, res, halvings);
     }
     p.nsplit = p.nsplit_p + p.nsplit_d;
     p.token_ub = dense_ub + blocks_ub * kgs;
@@ -1685,7 +1685,7 @@ size_t attn_workspace_bytes(int dense_ub, int blocks_ub, int Hq, int Hkv, int D,
         bytes = p.bytes;
     }
     const long long heads = static_cast<long long>(Hkv) * ((G + gp_for(G) - 1) / gp_for(G));
-    p.nsplit = valu_slots(units, heads, D, split_residency(D, G, meta_fp16, false, true), false);
+    p.nsplit = valu_slots(units, heads, D, split_residency(D, G, meta_fp16, false, true), 0);
     plan_layout(p, Hq, D);
     return std::max(bytes, p.bytes);
 }

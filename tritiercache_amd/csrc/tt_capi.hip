@@ -91,7 +91,7 @@ int check_common(int dense_count, int num_blocks, int Hq, int Hkv, int D, int kg
 int prepare(const float* Q, const float* dK, const float* dV, int dense_count, const int32_t* KP, const void* KS,
             const void* KZ, const int32_t* VP, const void* VS, const void* VZ, const int64_t* ids, int num_blocks,
             int Hq, int Hkv, int D, int kgs, int meta_fp16, bool want_mw, AttnInputs* in, AttnPlan* plan,
-            bool fewer = false) {
+            int halvings = 0) {
     int rc = check_common(dense_count, num_blocks, Hq, Hkv, D, kgs);
     if (rc) return rc;
     if (!Q) TT_FAIL(TT_ERR_INVALID_ARGUMENT, "Argument 'Q' pointer address is NULL.");
@@ -100,7 +100,7 @@ int prepare(const float* Q, const float* dK, const float* dV, int dense_count, c
     if (num_blocks > 0 && (!KP || !KS || !KZ || !VP || !VS || !VZ || !ids))
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "PBS arguments must be non-NULL when num_blocks > 0.");
     if (!plan) return TT_OK;
-    *plan = attn_plan(dense_count, num_blocks, Hq, Hkv, D, kgs, want_mw, meta_fp16, fewer);
+    *plan = attn_plan(dense_count, num_blocks, Hq, Hkv, D, kgs, want_mw, meta_fp16, halvings);
     if (want_mw && !logits_fit(Hq, plan->ld))
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "num_q_heads x tokens exceeds the 4 GiB logits buffer of the mean weights.");
     in->Q = Q;
@@ -128,12 +128,12 @@ enum Phase { kBoth, kPartials, kFinalize };
 int fused_impl(const float* Q, const float* dK, const float* dV, int dense_count, const int32_t* KP, const void* KS,
                const void* KZ, const int32_t* VP, const void* VS, const void* VZ, const int64_t* ids, int num_blocks,
                int Hq, int Hkv, int D, float* out, float* mw, int kgs, int meta_fp16, void* ws, size_t ws_bytes,
-               bool own_ws, Phase phase, int want_mw, hipStream_t s, bool fewer = false) {
+               bool own_ws, Phase phase, int want_mw, hipStream_t s, int halvings = 0) {
     AttnInputs in;
     AttnPlan plan;
     const bool logits = (phase == kBoth) ? (mw != nullptr) : (want_mw != 0);
     int rc = prepare(Q, dK, dV, dense_count, KP, KS, KZ, VP, VS, VZ, ids, num_blocks, Hq, Hkv, D, kgs, meta_fp16,
-                     logits, &in, &plan, fewer);
+                     logits, &in, &plan, halvings);
     if (rc) return rc;
     if (phase == kBoth && !out) TT_FAIL(TT_ERR_INVALID_ARGUMENT, "Argument 'attn_output' pointer address is NULL.");
     if (phase == kFinalize && !out && !mw)
@@ -303,11 +303,11 @@ int tt_fused_attention_decode_noalloc(const float* Q, const float* dense_K, cons
                      PBS_V_Scales, PBS_V_Zeroes, PBS_token_ids, num_blocks, num_q_heads, num_kv_heads, head_dim,
                      k_group_size, meta_fp16, mean_attn_weights != nullptr, &in, &plan);
     if (rc) return rc;
-    // a context whose logits all but fill the scratch: partials of half as many slots
-    const bool fewer = plan.bytes > kScratchBytes;
-    if (fewer)
+    // a context whose logits all but fill the scratch: partials of half as many slots, down to one per head
+    int halvings = 0;
+    while (plan.bytes > kScratchBytes && plan.nsplit_p == 0 && plan.nsplit > 1)
         plan = attn_plan(dense_count, num_blocks, num_q_heads, num_kv_heads, head_dim, k_group_size,
-                         mean_attn_weights != nullptr, meta_fp16, true);
+                         mean_attn_weights != nullptr, meta_fp16, ++halvings);
     if (plan.bytes > kScratchBytes)
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "tt_fused_attention_decode_noalloc: the call needs " +
                                              std::to_string(plan.bytes) + " bytes of scratch; the static scratch holds " +
@@ -319,7 +319,7 @@ int tt_fused_attention_decode_noalloc(const float* Q, const float* dense_K, cons
     return fused_impl(Q, dense_K, dense_V, dense_count, PBS_K_Packed, PBS_K_Scales, PBS_K_Zeroes, PBS_V_Packed,
                       PBS_V_Scales, PBS_V_Zeroes, PBS_token_ids, num_blocks, num_q_heads, num_kv_heads, head_dim,
                       attn_output, mean_attn_weights, k_group_size, meta_fp16, ws, kScratchBytes, false, kBoth, 0,
-                      as_stream(stream), fewer);
+                      as_stream(stream), halvings);
 }
 
 size_t tt_fused_attention_workspace_bytes(int dense_count, int num_blocks, int num_q_heads, int num_kv_heads,
