@@ -8,16 +8,13 @@
 // division and round-to-nearest-even give them, software F16C-equivalent
 // rounding. They run once per 16 evictions, or in bulk at prefill.
 #include "tt_quant_dev.h"
-
-#include <algorithm>
+#include "tt_quant_grid.h"
 
 namespace tt {
 
 namespace {
 
 constexpr int kMaxGridY = 65535;  // largest grid y extent
-// threads of a 1-D launch at most (a dispatch counts its work-items in 32 bits)
-constexpr long long kMaxThreads = 0xFFFFFF00LL;
 
 __device__ __forceinline__ float4 load_meta4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 load_meta4(const uint16_t* p) {
@@ -136,14 +133,13 @@ __global__ void __launch_bounds__(256) dequantize_k4_kernel(const int32_t* __res
 // 45.1 us (5.9 TB/s) against 85.7 with a word's 16 channels per thread, whose
 // stores leave 64 bytes between lanes; four quads per thread 47.8. (row, rem)
 // of a quad's word are stepped rather than divided anew.
-constexpr int kDeqVPer = 2;
 template <typename MetaT, bool NT>
 __global__ void __launch_bounds__(256) dequantize_v4_kernel(const int32_t* __restrict__ packed,
                                                             const MetaT* __restrict__ scale,
                                                             const MetaT* __restrict__ zero, float* __restrict__ out,
                                                             unsigned words, unsigned wpr) {
     // 64 words (256 quads) per workgroup and step
-    const size_t w0 = static_cast<size_t>(blockIdx.x) * (64 * kDeqVPer) + (threadIdx.x >> 2);
+    const size_t w0 = static_cast<size_t>(blockIdx.x) * kDeqVWords + (threadIdx.x >> 2);
     const int sh = 8 * (threadIdx.x & 3);
     unsigned row = static_cast<unsigned>(w0) / wpr, rem = static_cast<unsigned>(w0) - row * wpr;
     const unsigned drow = 64 / wpr, drem = 64 - drow * wpr;
@@ -226,7 +222,7 @@ int launch_quantize_k(const float* K, uint32_t* packed, void* scale, void* zero,
     if (num_blocks <= 0 || H * D <= 0) return TT_OK;
     // slices of whole blocks that a 1-D launch can hold
     const unsigned row = static_cast<unsigned>(H * D);
-    const int per = static_cast<int>(std::min<long long>(num_blocks, kMaxThreads / row));
+    const int per = quant_k_slice(num_blocks, row);
     const int words = kgs / 16;
     for (int b0 = 0; b0 < num_blocks; b0 += per) {
         const int nb = std::min(per, num_blocks - b0);
@@ -285,7 +281,7 @@ int launch_dequantize_k(const int32_t* packed, const void* scale, const void* ze
     if (num_blocks <= 0 || H * D <= 0) return TT_OK;
     const size_t meta4 = meta_fp16 ? 8 : 16;
     const long long items = static_cast<long long>(num_blocks) * (H * D / 4);
-    if (H * D % 4 == 0 && items <= kMaxThreads && aligned(packed, 16) && aligned(out, 16) && aligned(scale, meta4) &&
+    if (H * D % 4 == 0 && deq_k_wide_fits(items) && aligned(packed, 16) && aligned(out, 16) && aligned(scale, meta4) &&
         aligned(zero, meta4)) {
         const dim3 grid(static_cast<unsigned>((items + 255) / 256));
         const unsigned row = static_cast<unsigned>(H * D), n = static_cast<unsigned>(items);
@@ -322,8 +318,9 @@ int launch_dequantize_v(const int32_t* packed, const void* scale, const void* ze
     const long long n = static_cast<long long>(tokens) * H * (D / 16);
     if (n <= 0) return TT_OK;
     if (n > kMaxThreads) TT_FAIL(TT_ERR_INVALID_ARGUMENT, "dequantize_v: tokens x heads too large for one call");
-    if (aligned(out, 16)) {
-        const dim3 grid(static_cast<unsigned>((n + 64 * kDeqVPer - 1) / (64 * kDeqVPer)));
+    // (from 2^31 words on, 137 GB of output, the wide kernel's threads are too many for a dispatch)
+    if (aligned(out, 16) && deq_v_wide_fits(n)) {
+        const dim3 grid(static_cast<unsigned>(deq_v_wide_groups(n)));
         const unsigned words = static_cast<unsigned>(n), wpr = static_cast<unsigned>(D / 16);
         const auto launch = [&](auto kernel, auto meta) {
             using MetaT = decltype(meta);
