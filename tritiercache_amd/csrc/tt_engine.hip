@@ -1330,11 +1330,12 @@ int tt_engine_buffer(tt_engine* e, int which, void** p, int64_t* numel, int* es,
     clear_error();
     if (!e || !p || !numel || !es) TT_FAIL(TT_ERR_INVALID_ARGUMENT, "engine or output is NULL.");
     DeviceGuard dg(e->device);
-    // The tiers of fixed size need no counters from the device; their pending
-    // feedback is enqueued all the same.
+    // A reader may be on any stream, so every getter waits for what was enqueued on this one; the tiers of fixed size
+    // need no counters from the device besides.
     const bool fixed = (which >= 0 && which <= 10) || which == 18;
     int rc = fixed ? engine_flush(e, as_stream(stream)) : engine_sync_state(e, as_stream(stream));
     if (rc) return rc;
+    if (fixed) TT_HIP_CHECK(hipStreamSynchronize(as_stream(stream)));
     const int64_t kvs = static_cast<int64_t>(e->kvs), nb = fixed ? 0 : e->host_state[kLogicalAlloc], ch = e->chunk;
     const int msz = static_cast<int>(e->msz());
     if (nb > e->cap_blocks) TT_FAIL(TT_ERR_RUNTIME, "packed store smaller than its logical allocation.");
