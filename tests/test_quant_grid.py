@@ -20,7 +20,9 @@ def grid(tmp_path_factory):
                              "int k_slice(int nb, long long row) { return tt::quant_k_slice(nb, row); }\n"
                              "int k_fits(long long q) { return tt::deq_k_wide_fits(q); }\n"
                              "int v_fits(long long w) { return tt::deq_v_wide_fits(w); }\n"
-                             "long long v_groups(long long w) { return tt::deq_v_wide_groups(w); }\n}\n")
+                             "long long v_groups(long long w) { return tt::deq_v_wide_groups(w); }\n"
+                             "int k_streams(long long v, int kgs, int f) { return tt::deq_k_streams(v, kgs, f); }\n"
+                             "int v_streams(long long v, int d, int f) { return tt::deq_v_streams(v, d, f); }\n}\n")
     subprocess.run(["g++", "-shared", "-fPIC", "-std=c++17", "-I", CSRC, str(d / "g.cpp"), "-o", str(d / "g.so")],
                    check=True)
     L = ctypes.CDLL(str(d / "g.so"))
@@ -55,3 +57,14 @@ def test_quantize_k_slices_cover_the_blocks(grid, row):
         assert 1 <= per <= blocks and (per * row + 255) // 256 * 256 <= LIMIT
         # a slice is as large as a dispatch allows, so the launches are few and cover every block
         assert per == blocks or ((per + 1) * row + 255) // 256 * 256 > LIMIT - 256
+
+
+@pytest.mark.parametrize("fp16", [0, 1])
+@pytest.mark.parametrize("kgs,d", [(16, 64), (32, 80), (16, 256)])
+def test_streaming_stores_start_past_the_last_level_cache(grid, kgs, d, fp16):
+    for mib in range(64, 512):
+        values, m = (mib << 20) // 4 // (kgs * d) * kgs * d, 2 if fp16 else 4
+        total = lambda per: 4 * values + values // 4 + 2 * m * (values // per)  # noqa: E731
+        v = ctypes.c_longlong(values)
+        assert bool(grid.k_streams(v, kgs, fp16)) == (total(kgs) > (280 if fp16 else 256) << 20)
+        assert bool(grid.v_streams(v, d, fp16)) == (total(d) > 256 << 20)

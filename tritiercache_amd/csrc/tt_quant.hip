@@ -29,11 +29,6 @@ __device__ __forceinline__ void store4(float* p, const float4 v) {
     else
         *reinterpret_cast<float4*>(p) = v;
 }
-// Outputs from 256 MB (what the last-level cache holds) go out as non-temporal
-// stores: 268 MB of K (V) take 47.9 (45.1) us with them and 52.7 (65.3)
-// without, 134 MB 24.8 (22.5) against 22.4 (23.1), and a smaller output stays
-// cached for its reader.
-inline bool deq_streams(const long long values) { return values * 4 >= (256LL << 20); }
 inline bool aligned(const void* p, const size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
 // One thread per (block, head, channel), flat over all blocks, so that short
@@ -290,7 +285,7 @@ int launch_dequantize_k(const int32_t* packed, const void* scale, const void* ze
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, packed, static_cast<const MetaT*>(scale),
                                static_cast<const MetaT*>(zero), out, row, n, kgs);
         };
-        const bool nt = deq_streams(static_cast<long long>(num_blocks) * kgs * row);
+        const bool nt = deq_k_streams(static_cast<long long>(num_blocks) * kgs * row, kgs, meta_fp16);
         if (meta_fp16)
             nt ? launch(dequantize_k4_kernel<uint16_t, true>, uint16_t{})
                : launch(dequantize_k4_kernel<uint16_t, false>, uint16_t{});
@@ -327,7 +322,7 @@ int launch_dequantize_v(const int32_t* packed, const void* scale, const void* ze
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, packed, static_cast<const MetaT*>(scale),
                                static_cast<const MetaT*>(zero), out, words, wpr);
         };
-        const bool nt = deq_streams(16 * n);
+        const bool nt = deq_v_streams(16 * n, D, meta_fp16);
         if (meta_fp16)
             nt ? launch(dequantize_v4_kernel<uint16_t, true>, uint16_t{})
                : launch(dequantize_v4_kernel<uint16_t, false>, uint16_t{});

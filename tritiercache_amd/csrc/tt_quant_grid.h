@@ -1,6 +1,6 @@
-// tt_quant_grid.h -- launch sizes of the quantisers and dequantisers, host
-// arithmetic only. A dispatch counts its work-items in 32 bits, so every
-// launch's grid times 256 threads stays within kMaxThreads.
+// tt_quant_grid.h -- launch sizes and choice of stores of the quantisers and
+// dequantisers, host arithmetic only. A dispatch counts its work-items in 32
+// bits, so every launch's grid times 256 threads stays within kMaxThreads.
 #pragma once
 
 #include <algorithm>
@@ -24,5 +24,24 @@ constexpr int kDeqVPer = 2;
 constexpr long long kDeqVWords = 64 * kDeqVPer;
 inline long long deq_v_wide_groups(const long long words) { return (words + kDeqVWords - 1) / kDeqVWords; }
 inline bool deq_v_wide_fits(const long long words) { return 256 * deq_v_wide_groups(words) <= kMaxThreads; }
+
+// Outputs go out as non-temporal stores where they and the tiers together
+// exceed the last-level cache (256 MiB), and stay cached for their reader
+// below. Over six shapes at outputs of 208 to 320 MB the two cross there for V
+// (per launch, plain against non-temporal, tiers and output in MiB: 242 36.9
+// against 39.8 us, 259 46.3 against 42.2, 276 64.3 against 45.6) and for K with
+// f32 metadata (252 39.4 against 43.2, 261 47.8 against 43.9, 288 56.0 against
+// 48.1), and at 261 to 300 for K with f16 metadata (262 43.3 against 45.8, 280 48.3
+// against 48.2, 298 56.2 against 51.7; head_dim 128 in blocks of 16: 288 53.0
+// against 54.5, 306 58.1 against 57.5).
+inline long long deq_bytes(const long long values, const int per_meta, const int meta_fp16) {
+    return 4 * values + values / 4 + 2 * (meta_fp16 ? 2 : 4) * (values / per_meta);
+}
+inline bool deq_k_streams(const long long values, const int kgs, const int meta_fp16) {
+    return deq_bytes(values, kgs, meta_fp16) > ((meta_fp16 ? 280LL : 256LL) << 20);
+}
+inline bool deq_v_streams(const long long values, const int D, const int meta_fp16) {
+    return deq_bytes(values, D, meta_fp16) > (256LL << 20);
+}
 
 }  // namespace tt
