@@ -22,6 +22,7 @@
 //                       engine's decayed score feedback (cache_engine.cpp:
 //                       511-540).
 #include "tt_attn.h"
+#include "tt_attn_line.h"
 
 #include <algorithm>
 #include <atomic>
@@ -1345,9 +1346,6 @@ int launch_batched_meta(const BatchArgs& b, unsigned wgs, int meta_fp16, hipStre
 
 inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
-int gp_for(int G) { return G >= 8 ? 8 : (G > 4 ? 8 : (G > 2 ? 4 : G)); }
-
-
 template <typename MetaT>
 const void* packed_kernel_ptr(int gp, bool pair) {
     if (pair) {
@@ -1456,38 +1454,6 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
                         int meta_fp16, bool pair, int halvings, bool valu);
 }  // namespace
 
-namespace {
-// Units (16-token tiles of either kind) per KV head up to which the VALU kernel
-// serves the head dims of the matrix-core kernel too. At short contexts a
-// launch is one chain of latencies, and the VALU kernel's is shorter: no
-// lay-out in LDS, no coefficients, a unit per wave. Its arithmetic grows with
-// units x query heads x channels, so the line is a number of units x heads per
-// CU for each group size and head dim, below the point where the matrix cores
-// win with blocks of 32 tokens. It was measured with the waves per SIMD that
-// the resource test of this kernel asks for (another register count moves the
-// times, not the line). Partials per launch, VALU against matrix cores, at
-// units x heads per CU:
-//   one head per group of 128 (line at 35): 32/32 heads at 2k (18) 6.7 against
-//     8.9 us, at 4k (32) 9.9 against 11.9, at 5k (39) 10.2 against 10.8, at
-//     6k (47) 12.5 against 12.0;
-//   two (16): 16/8 heads at 4k (8) 5.7 against 7.9, at 8k (16) 7.6 against 7.9;
-//   four (4.5): 32/8 heads at 580 (1.1) 5.5 against 5.9, at 2k (4.0) 5.9 against
-//     7.0, at 2.3k (4.5) 7.0 against 7.0, at 3k (5.9) 7.3 against 7.2;
-//   more: 28/4 heads at 1k (1) 7.4 against 6.2;
-//   head_dim 64: one (28): 64/64 heads at 1.5k (24) 6.9 against 8.2, at 2.6k
-//     (41) 9.8 against 9.6; two (20): 32/16 heads at 5k (20) 7.2 against 8.5;
-//     four (16): 32/8 heads at 6k (12) 6.9 against 7.5, at 8k (16) 8.0 against
-//     8.0; more (1.5): 14/2 heads at 3k (1.5) 6.2 against 6.4.
-long long short_units(int Hq, int Hkv, int D, int meta_fp16) {
-    const int G = Hq / Hkv, gp = gp_for(G);
-    const int halves = D == 64 ? (gp == 1 ? 56 : gp == 2 ? 40 : gp == 4 ? 32 : 3)
-                               : (gp == 1 ? 70 : gp == 2 ? 32 : gp == 4 ? 9 : 0);
-    const long long heads = static_cast<long long>(Hkv) * ((G + gp - 1) / gp);
-    return static_cast<long long>(split_residency(D, G, meta_fp16, false, true).cus) * halves / (2 * heads);
-}
-bool use_matrix_cores(int D, int Hkv) { return use_packed_kernel(D) || (D == 64 && Hkv % 2 == 0); }
-}  // namespace
-
 // Head_dim 64 with an even number of KV heads runs as half as many heads of
 // head_dim 128 on the matrix-core kernel: KV heads 2j and 2j + 1 sit next to
 // each other in every tier (K words and scale / zero per block, V words per
@@ -1497,8 +1463,8 @@ bool use_matrix_cores(int D, int Hkv) { return use_packed_kernel(D) || (D == 64 
 AttnPlan attn_plan(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int kgs, bool need_logits, int meta_fp16,
                    int halvings) {
     const bool pair = D == 64 && Hkv % 2 == 0;
-    const long long units = (static_cast<long long>(dense_ub) + 15) / 16 + static_cast<long long>(blocks_ub) * (kgs / 16);
-    const bool valu = !use_matrix_cores(D, Hkv) || units <= short_units(Hq, Hkv, D, meta_fp16);
+    const int cus = split_residency(D, Hq / Hkv, meta_fp16, false, true).cus;
+    const bool valu = use_valu(dense_ub, blocks_ub, Hq, Hkv, D, kgs, cus);
     if (pair && !valu) {
         AttnPlan p = attn_plan_impl(dense_ub, blocks_ub, Hq, Hkv / 2, kMfD, kgs, need_logits, meta_fp16, true, halvings, false);
         p.pair64 = true;
@@ -1560,8 +1526,7 @@ AttnPlan attn_plan_impl(int dense_ub, int blocks_ub, int Hq, int Hkv, int D, int
     AttnPlan p;
     const int W = kgs / 16;
     const int G = Hq / Hkv;
-    const int chunks = (G + gp_for(G) - 1) / gp_for(G);
-    const long long heads = static_cast<long long>(Hkv) * chunks;
+    const long long heads = head_chunks(Hq, Hkv);
     const Residency res = split_residency(D, G, meta_fp16, pair, valu);
     const long long resident = static_cast<long long>(res.cus) * res.per_cu;
     const long long per_head = std::max<long long>(1, (resident + heads - 1) / heads);
@@ -1674,18 +1639,17 @@ size_t attn_workspace_bytes(int dense_ub, int blocks_ub, int Hq, int Hkv, int D,
     p.logits = need_logits;
     size_t bytes = 0;
     long long units = valu_units(dense_ub, blocks_ub, D, kgs);
+    const Residency valu = split_residency(D, G, meta_fp16, false, true);
     if (use_matrix_cores(D, Hkv)) {
-        units = std::min(units, short_units(Hq, Hkv, D, meta_fp16));
+        units = std::min(units, short_units(Hq, Hkv, D, valu.cus));
         const bool pair = D == 64;
-        const int g = pair ? 2 * G : G, hkv = pair ? Hkv / 2 : Hkv;
-        const long long heads = static_cast<long long>(hkv) * ((g + gp_for(g) - 1) / gp_for(g));
-        p.nsplit = static_cast<int>(matrix_slots(matrix_units(dense_ub, blocks_ub, kgs), heads,
-                                                 split_residency(kMfD, g, meta_fp16, pair)));
+        p.nsplit = static_cast<int>(matrix_slots(matrix_units(dense_ub, blocks_ub, kgs),
+                                                 head_chunks(Hq, pair ? Hkv / 2 : Hkv),
+                                                 split_residency(kMfD, pair ? 2 * G : G, meta_fp16, pair)));
         plan_layout(p, Hq, kMfD);
         bytes = p.bytes;
     }
-    const long long heads = static_cast<long long>(Hkv) * ((G + gp_for(G) - 1) / gp_for(G));
-    p.nsplit = valu_slots(units, heads, D, split_residency(D, G, meta_fp16, false, true), 0);
+    p.nsplit = valu_slots(units, head_chunks(Hq, Hkv), D, valu, 0);
     plan_layout(p, Hq, D);
     return std::max(bytes, p.bytes);
 }
@@ -1837,13 +1801,11 @@ BatchPlan batch_plan(const tt_decode_seq* seqs, int nseq, int Hq, int Hkv, int D
     p.nseq = nseq;
     const int W = kgs / 16;
     const int G = Hq / Hkv;
-    const int gp = gp_for(G);
-    const long long heads = static_cast<long long>(Hkv) * ((G + gp - 1) / gp);
+    const long long heads = head_chunks(Hq, Hkv);
     const Residency res = split_residency(D, G, meta_fp16);
     // Slots per head that fill the device once; fewer when the batch is small
     // (at least ~8 units of work per slot, as for one sequence).
     const long long round = std::max<long long>(1, static_cast<long long>(res.cus) * res.per_cu / heads);
-    constexpr long long kDenseTileCost = 4;
     constexpr long long kBatchSlotUnits = 40;  // work units per slot below which another round does not pay
     long long units[kMaxBatchSeqs], dunits[kMaxBatchSeqs], total = 0, mean_blocks = 0;
     for (int i = 0; i < nseq; ++i) {
