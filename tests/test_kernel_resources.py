@@ -74,3 +74,8 @@ def test_short_context_kernel_keeps_its_waves(resources, cpl, gp):
     assert len(found) == 2, sorted(found)  # fp32 and fp16 metadata
     for name, res in found.items():
         assert res["ScratchSize"] == 0 and res["Occupancy"] >= SPLIT_WAVES[cpl, gp], (name, res)
+
+
+def test_batched_finalize_keeps_four_waves(resources):
+    found = [v for k, v in resources.items() if "attn_finalize_batched_kernel" in k]
+    assert len(found) == 1 and found[0]["ScratchSize"] == 0 and found[0]["Occupancy"] >= 4, found

@@ -696,9 +696,10 @@ __device__ __forceinline__ void fin_merge_head(const FinArgs& a, const int h, co
         float4 v[kMergeU];
 #pragma unroll
         for (int u = 0; u < kMergeU; ++u) {
+            // (past the last split no load and zeros: a re-read sum may be infinite, and a zero factor makes a NaN of it)
             v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (u * groups < nj)  // splits past the last re-read it and are not added
-                v[u] = *reinterpret_cast<const float4*>(base + static_cast<size_t>(j0 + min(g + u * groups, nj - 1)) * a.D);
+            const int j = g + u * groups;
+            if (j < nj) v[u] = *reinterpret_cast<const float4*>(base + static_cast<size_t>(j0 + j) * a.D);
         }
         // the whole block's statistics in every wave, so that no wave waits for another
         const float Mn = fmaxf(M, wave_max(fmaxf(fmaxf(st[0].x, st[1].x), fmaxf(st[2].x, st[3].x))));
@@ -722,17 +723,9 @@ __device__ __forceinline__ void fin_merge_head(const FinArgs& a, const int h, co
             A.z = __builtin_fmaf(f, x.z, A.z);
             A.w = __builtin_fmaf(f, x.w, A.w);
         };
-        // (a re-read split is replaced by zeros rather than given a zero factor alone: its sums may be infinite;
-        // threads past the last whole group add what nothing reads)
 #pragma unroll
-        for (int u = 0; u < kMergeU; ++u) {
-            if (u * groups < nj) {
-                const int j = g + u * groups;
-                const bool in = j < nj;
-                add(own[min(j, nj - 1)], make_float4(in ? v[u].x : 0.0f, in ? v[u].y : 0.0f, in ? v[u].z : 0.0f,
-                                                     in ? v[u].w : 0.0f));
-            }
-        }
+        for (int u = 0; u < kMergeU; ++u)
+            if (u * groups < nj) add(own[min(g + u * groups, nj - 1)], v[u]);
         // splits beyond kMergeU per group in this block of 256 (groups < 16 only)
         for (int j = g + kMergeU * groups; g < groups && j < nj; j += groups)
             add(own[j], *reinterpret_cast<const float4*>(base + static_cast<size_t>(j0 + j) * a.D));
