@@ -207,7 +207,10 @@ TT_API int tt_attention_finalize_deferred(const float* Q, int dense_count, int n
  * tier tables and lengths, in one split-K launch plus one merge launch (head_dim
  * 128; other head dims run the sequences one after another). No counterpart
  * in the reference, whose callers run fused_attention_decode (bindings.cpp:
- * 99-178) once per sequence; each sequence's result is that call's result.
+ * 99-178) once per sequence; each sequence's result is that call's result up to
+ * the order and the operands of its sums (a batch keeps short contexts of
+ * head_dim 128 on the matrix cores, a single call runs them in FP32; both stay
+ * within the kernels' tolerance).
  *
  * One tt_decode_seq holds the arguments of tt_fused_attention_decode for one
  * sequence (all device pointers; mean_attn_weights may be NULL, the PBS
@@ -329,8 +332,9 @@ TT_API int tt_engine_buffer_bytes(tt_engine* e, size_t* out, void* stream);
  * 11 PBS_K_Packed 12 PBS_K_Scales 13 PBS_K_Zeroes 14 PBS_V_Packed 15 PBS_V_Scales
  * 16 PBS_V_Zeroes 17 PBS_token_ids 18 global_attn_scores 19 mean attention
  * weights of the last step [visible] (no reference getter). PBS buffers are sized
- * by pbs_allocated_blocks (synchronises `stream`). The pointers stay valid
- * until the physical PBS capacity grows (only past max_seq_len tokens). */
+ * by pbs_allocated_blocks. Every call runs the engine's pending feedback and
+ * synchronises `stream`, so the pointer can be read from any stream. It stays
+ * valid until the physical PBS capacity grows (only past max_seq_len tokens). */
 TT_API int tt_engine_buffer(tt_engine* e, int which, void** dev_ptr, int64_t* numel, int* elem_size,
                      void* stream);
 

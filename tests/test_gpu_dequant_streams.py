@@ -1,6 +1,7 @@
 """The dequantisers on both sides of the size from which their stores bypass the caches, with a ragged last workgroup:
 bit for bit what the narrow kernels write (an output one float past a 16-byte boundary), which are held to the oracle
-at small sizes; the first and last block, token and 65,536th block against the oracle too."""
+at small sizes; the first and last block, token and 65,536th block against the oracle too (the narrow K launch is
+sliced after 65,535 blocks)."""
 import numpy as np
 import pytest
 import torch

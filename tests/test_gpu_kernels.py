@@ -146,8 +146,9 @@ def test_quantize_v_unaligned_rows_vs_oracle(C, oracle, fp16):
 
 @pytest.mark.parametrize("fp16", [False, True])
 def test_k_block_calls_past_the_grid_y_extent(C, oracle, fp16):
-    """One quantize_k / dequantize_k call over more blocks than a grid's y extent (65535): the launches
-    are sliced, and the blocks on both sides of the seam, the first and the last match the oracle."""
+    """One quantize_k / dequantize_k call over more blocks than a grid's y extent (65535), on which the flat launches of
+    both do not depend (only the narrow dequantiser's is sliced there): the blocks on both sides, the first and the
+    last match the oracle."""
     import ctypes as ct
     from tritiercache_amd import _lib
 

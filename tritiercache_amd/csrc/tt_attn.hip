@@ -223,17 +223,19 @@ __device__ __forceinline__ float rows_sum4(const float (&v)[4]) {
 }
 
 // CPL: channels per lane (head_dim / 16). GP: query heads per workgroup
-// (padded to a power of two; heads past the group are zero and never stored).
+// (padded to a power of two; heads past the group repeat its last one and are
+// never stored).
 //
 // Each wave owns a contiguous share of its KV head's units: FP32 units of
 // split_unit_tokens, then 16-token packed tiles, counted alike (an FP32 unit
 // holds more bytes and needs fewer instructions; at two, four or eight tiles
-// per FP32 unit the launches took the same or up to 15% longer). Share
-// wave nsplit_d + split, so that every workgroup holds both kinds. Lane (row group tg, channel lane cp) holds channels
-// cp CPL .. + CPL - 1 of tokens tg, tg + 4, ...: a K word shifted by 2 tg has
-// those tokens' codes in the low bits of its four bytes, so one mask and four
-// byte conversions unpack them. The row's logits come from a DPP sum over its
-// 16 lanes; V is unpacked after the softmax, when K is no longer live.
+// per FP32 unit the launches took the same or up to 15% longer). Wave w of
+// workgroup `split` has share w nsplit_d + split, so that every workgroup
+// holds both kinds. Lane (row group tg, channel lane cp) holds channels cp CPL
+// .. + CPL - 1 of tokens tg, tg + 4, ...: a K word shifted by 2 tg has those
+// tokens' codes in the low bits of its four bytes, so one mask and four byte
+// conversions unpack them. The row's logits come from a DPP sum over its 16
+// lanes; V is unpacked after the softmax, when K is no longer live.
 //
 // A wave has one to three units, so the launch is a chain: arguments, query
 // and first unit's loads, arithmetic (about 850 VALU instructions per packed
@@ -282,7 +284,7 @@ __device__ __forceinline__ void split_body(const SplitArgs& a, const int split, 
     const int Hkv = in.Hkv;
 
     // The wave's share of the Td FP32 units and Tp packed tiles.
-        const int part = wave * a.nsplit_d + split, parts = 4 * a.nsplit_d;
+    const int part = wave * a.nsplit_d + split, parts = 4 * a.nsplit_d;
     const int lo = part_begin(Td + Tp, part, parts), hi = part_begin(Td + Tp, part + 1, parts);
     const int d_begin = min(lo, Td), d_end = min(hi, Td);
     const int p_begin = max(lo - Td, 0), p_end = max(hi - Td, 0);
@@ -1735,8 +1737,9 @@ int fin_mean_wgs(const AttnPlan& plan, const bool weights) {
     return (blocks + per_wg - 1) / per_wg;
 }
 
+// The merge's 256 floats per wave; a mean-weight workgroup's two statistics per head and a sum per wave and token.
 size_t fin_lds_bytes(const int Hq) {
-    return sizeof(float) * std::max<size_t>(8 + 4 * 256, 2 * static_cast<size_t>(Hq) + 256 * 4);
+    return sizeof(float) * std::max<size_t>(4 * 256, 2 * static_cast<size_t>(Hq) + 4 * kMeanTokensLong);
 }
 }  // namespace
 
@@ -1973,7 +1976,7 @@ int batch_launch(const BatchPlan& plan, const tt_decode_seq* seqs_dev, int Hq, i
     std::memcpy(f.slot_base, plan.slot_base, sizeof(f.slot_base));
     std::memcpy(f.tok_base, plan.tok_base, sizeof(f.tok_base));
     std::memcpy(f.mean_base, plan.mean_base, sizeof(f.mean_base));
-    const size_t lds = sizeof(float) * std::max<size_t>(8 + 4 * 256, 2 * static_cast<size_t>(Hq) + 256 * 4);
+    const size_t lds = fin_lds_bytes(Hq);
     const long long fwgs = static_cast<long long>(plan.nseq) * Hq * f.msl + plan.mean_base[plan.nseq];
     hipLaunchKernelGGL(attn_finalize_batched_kernel, dim3(static_cast<unsigned>(fwgs)), dim3(256), lds, stream, f);
     TT_LAUNCH_CHECK();
