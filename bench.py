@@ -153,7 +153,7 @@ PMC_TRAFFIC_MD = os.path.join(ROOT, "profiles", "attn_packed_kernel_llama3-8b-32
 DEFER_MIN_LAYERS = 16  # steps of at least this many layers time the deferred-mean-weights layout
 
 
-KERNEL_SOURCES = ("tt_attn.hip", "tt_attn_mfma.h", "tt_attn.h", "tt_common.h")
+KERNEL_SOURCES = ("tt_attn.hip", "tt_attn_mfma.h", "tt_attn.h", "tt_attn_line.h", "tt_common.h")
 
 
 def kernel_source_digest():

@@ -23,7 +23,7 @@ def _scores(kind, n):
 
 
 @pytest.mark.parametrize("kind", ["zeros", "few", "signed", "decayed"])
-@pytest.mark.parametrize("n", [1, 64, 1025, 16385, 32768, 32769, 40001])
+@pytest.mark.parametrize("n", [1, 64, 1025, 16385, 28672, 28673, 32768, 32769, 40001])
 def test_threshold_is_exact(oracle, n, kind):
     from tritiercache_amd import _C
 

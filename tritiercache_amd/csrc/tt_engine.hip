@@ -58,11 +58,13 @@ __global__ void __launch_bounds__(256) append_row_kernel(const float* __restrict
 //
 // What it waits for is one read of the scores by one CU and the LDS atomics:
 // scores share few leading digits (after a prefill they are all zero), so a
-// wave adds the lanes that hold its first lane's digit in one atomic. 16k
-// zeros after a prefill: 18 us (50 with an atomic per lane and a read per
-// pass). The spread selection's six launches take about twice the 30 us of
-// 32k candidates here.
-constexpr int kThrPer = 32;
+// wave adds the lanes that hold its first lane's digit in one atomic. (The loads
+// are plain: with the keys formed in their branches each waited for itself.)
+// An ingest with a refresh, one workgroup against the spread selection's six
+// launches: 15k zeros 20.7 against 28.5 us (52 with an atomic per lane and a
+// read per pass), 26k 27.7 against 29.1, 29k 29.5 against 29.1, 32k 31.5 against
+// 29.1; 26k decayed scores 18.4 against 23.3, 32k 20.7 against 23.3.
+constexpr int kThrPer = 28;
 constexpr int kThrOneWg = 1024 * kThrPer;
 
 __device__ __forceinline__ unsigned int wave_incl_scan(unsigned int x) {
@@ -75,8 +77,8 @@ __device__ __forceinline__ unsigned int wave_incl_scan(unsigned int x) {
     return x;
 }
 
-__device__ __forceinline__ unsigned int order_key(const float v) {
-    const unsigned int u = __float_as_uint(v);
+// Order-preserving image of a float's bits.
+__device__ __forceinline__ unsigned int order_key(const unsigned int u) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
@@ -108,8 +110,10 @@ __global__ void __launch_bounds__(1024) threshold_kernel(const float* __restrict
 #pragma unroll
     for (int j = 0; j < kThrPer; ++j) {
         const int i = j * 1024 + tid;
-        key[j] = i < n ? order_key(g[i]) : 0u;
+        key[j] = i < n ? __float_as_uint(g[i]) : 0u;
     }
+#pragma unroll
+    for (int j = 0; j < kThrPer; ++j) key[j] = order_key(key[j]);
     for (int pass = 0; pass < 3; ++pass) {
         const int bits = pass < 2 ? 11 : 10;
         const int shift = pass == 0 ? 21 : (pass == 1 ? 10 : 0);
@@ -151,8 +155,9 @@ __global__ void __launch_bounds__(1024) threshold_kernel(const float* __restrict
 
 // The same selection spread over many workgroups: per pass, thr_hist_kernel
 // adds the digit histogram of the candidates that match the prefix found so
-// far into a global histogram (LDS histogram per workgroup, then one atomic
-// per non-empty bin), and thr_select_kernel (one workgroup) finds the digit
+// far into a global histogram (LDS histogram per workgroup, an atomic per lane:
+// adding a wave's common digit at once took 1 to 2 us more over the passes; then
+// one atomic per non-empty bin), and thr_select_kernel (one workgroup) finds the digit
 // where the running count passes k, narrows prefix / mask / k, clears the
 // histogram for the next pass and, after the last pass, writes the threshold.
 // Selection state (`ts`): hist[2048], then prefix, mask, k; all zero between
@@ -174,15 +179,17 @@ __global__ void __launch_bounds__(256) thr_hist_kernel(const float* __restrict__
     const unsigned int prefix = ts[2048], mask = ts[2049];
     const int stride = gridDim.x * 256 * kThrHistPer;
     for (int base = blockIdx.x * 256 * kThrHistPer; base < n; base += stride) {
-        unsigned int key[kThrHistPer];
+        unsigned int u[kThrHistPer];
 #pragma unroll
         for (int j = 0; j < kThrHistPer; ++j) {
             const int i = base + j * 256 + tid;
-            key[j] = i < n ? order_key(g[i]) : 0u;
+            u[j] = i < n ? __float_as_uint(g[i]) : 0u;
         }
 #pragma unroll
-        for (int j = 0; j < kThrHistPer; ++j)
-            hist_add(hist, (key[j] >> shift) & dm, base + j * 256 + tid < n && (key[j] & mask) == prefix);
+        for (int j = 0; j < kThrHistPer; ++j) {
+            const unsigned int key = order_key(u[j]);
+            if (base + j * 256 + tid < n && (key & mask) == prefix) atomicAdd(&hist[(key >> shift) & dm], 1u);
+        }
     }
     __syncthreads();
     for (int i = tid; i < 2048; i += 256)
