@@ -66,3 +66,17 @@ def test_codes_and_stores_at_the_edges(C, oracle, h, d, nb, kgs, fp16, shift):
     out.zero_()
     C.dequantize_v(vp, vs, vz, out, n, h, d, meta)
     assert same_bits(host(out).reshape(n, h, d), oracle.dequantize_v(p, s, z, n, h, d, fp16))
+
+
+# more than a wave per SIMD, where the quantisers' codes come from the reciprocal and the K stores are wide
+@pytest.mark.parametrize("h,d,nb,kgs,fp16", [(1, 16, 4099, 16, False), (3, 80, 277, 32, True), (2, 256, 131, 16, False),
+                                             (5, 96, 139, 16, True), (1, 1040, 67, 16, False), (3, 18, 1217, 16, False)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_codes_and_stores_at_the_edges_of_large_launches(C, oracle, h, d, nb, kgs, fp16, shift):
+    test_codes_and_stores_at_the_edges(C, oracle, h, d, nb, kgs, fp16, shift)
+
+
+@pytest.mark.parametrize("blocks", [255, 256, 257])
+def test_both_sides_of_a_wave_per_simd(C, oracle, blocks):
+    """65,536 threads and a block less and more: 2 heads of 128 channels in blocks of 32 (K), V rows of 8 words."""
+    test_codes_and_stores_at_the_edges(C, oracle, 2, 128, blocks, 32, True, 0)

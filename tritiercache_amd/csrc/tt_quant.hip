@@ -40,8 +40,9 @@ inline bool aligned(const void* p, const size_t n) { return (reinterpret_cast<ui
 //
 // One f32 read per value is what bounds it: 134 MB in 23.4 us (5.7 TB/s; 25.8
 // us with a grid row per block and a division per value). Two and four
-// channels per thread (8- and 16-byte loads) took 24.2 and 26.3 us.
-template <typename MetaT>
+// channels per thread (8- and 16-byte loads) took 24.2 and 26.3 us. Launches of
+// at most a wave per SIMD divide every value (see quant_codes).
+template <typename MetaT, bool FAST>
 __global__ void __launch_bounds__(256) quantize_k_kernel(const float* __restrict__ K, uint32_t* __restrict__ packed,
                                                          MetaT* __restrict__ scale, MetaT* __restrict__ zero,
                                                          unsigned items, unsigned row, unsigned D, int kgs,
@@ -51,7 +52,7 @@ __global__ void __launch_bounds__(256) quantize_k_kernel(const float* __restrict
     const unsigned b = item / row, hc = item - b * row, c = hc % D;
     const size_t ob = static_cast<size_t>(b) + (base_dev ? *base_dev : 0);
     const size_t mi = ob * row + hc;
-    quant_k_channel<MetaT>(K + static_cast<size_t>(b) * kgs * row + hc, row, kgs, c < (D / 8) * 8, scale + mi,
+    quant_k_channel<MetaT, FAST>(K + static_cast<size_t>(b) * kgs * row + hc, row, kgs, c < (D / 8) * 8, scale + mi,
                            zero + mi, packed + ob * (kgs / 16) * row + hc, row);
 }
 
@@ -59,7 +60,7 @@ __global__ void __launch_bounds__(256) quantize_k_kernel(const float* __restrict
 // on an aligned group of `group` lanes (a power of two, at most 64, so the
 // group lies in one wave; lanes past D / 16 only pad the min/max tree), the
 // loads of a row coalesced. D % 16 == 0 (checked by the host).
-template <typename MetaT>
+template <typename MetaT, bool FAST>
 __global__ void __launch_bounds__(256) quantize_v_kernel(const float* __restrict__ V, int32_t* __restrict__ packed,
                                                          MetaT* __restrict__ scale, MetaT* __restrict__ zero,
                                                          int tokens, int H, int D, int group,
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(256) quantize_v_kernel(const float* __restrict
     const int t = r / H, h = r % H;
     const int ot = t + (base_dev ? (*base_dev) * tokens_per_block : 0);
     const size_t mi = static_cast<size_t>(ot) * H + h;
-    quant_v_row_lanes<MetaT>(V + static_cast<size_t>(t) * H * D + static_cast<size_t>(h) * D, w, wpr, group,
+    quant_v_row_lanes<MetaT, FAST>(V + static_cast<size_t>(t) * H * D + static_cast<size_t>(h) * D, w, wpr, group,
                              scale + mi, zero + mi, packed + mi * wpr);
 }
 
@@ -95,7 +96,9 @@ __global__ void __launch_bounds__(256) quantize_v_serial_kernel(const float* __r
 // K with four channels per thread: a wave stores 1 KB runs of a token's row
 // (16 bytes per lane). Threads are laid flat over (block, channel quad), so
 // short rows leave no lane idle. 268 MB: 47.9 us (5.6 TB/s) against 66 with
-// one channel per thread.
+// one channel per thread, 20 MB in blocks of 32 5.2 against 6.2. Up to a wave
+// per SIMD with one channel per thread that is the shorter chain (2 MB in
+// blocks of 32 3.0 us against 3.1, 0.5 MB 2.7 against 2.9).
 template <typename MetaT, bool NT>
 __global__ void __launch_bounds__(256) dequantize_k4_kernel(const int32_t* __restrict__ packed,
                                                             const MetaT* __restrict__ scale,
@@ -108,10 +111,8 @@ __global__ void __launch_bounds__(256) dequantize_k4_kernel(const int32_t* __res
     const size_t mi = static_cast<size_t>(b) * row + c;
     const float4 s = load_meta4(scale + mi), z = load_meta4(zero + mi);
     const int words = kgs / 16;
-    for (int w = 0; w < words; ++w) {
-        const size_t tok0 = (static_cast<size_t>(b) * words + w) * 16;
-        const int4 p = *reinterpret_cast<const int4*>(packed + (static_cast<size_t>(b) * words + w) * row + c);
-        float* o = out + tok0 * row + c;
+    auto put = [&](const int w, const int4 p) {
+        float* o = out + (static_cast<size_t>(b) * words + w) * 16 * row + c;
 #pragma unroll
         for (int st = 0; st < 16; ++st) {
             auto x = [&](const int v, const float sc, const float ze) {
@@ -120,6 +121,19 @@ __global__ void __launch_bounds__(256) dequantize_k4_kernel(const int32_t* __res
             store4<NT>(o + static_cast<size_t>(st) * row,
                    make_float4(x(p.x, s.x, z.x), x(p.y, s.y, z.y), x(p.z, s.z, z.z), x(p.w, s.w, z.w)));
         }
+    };
+    const int32_t* src = packed + static_cast<size_t>(b) * words * row + c;
+    if constexpr (NT) {
+        for (int w = 0; w < words; ++w) put(w, *reinterpret_cast<const int4*>(src + static_cast<size_t>(w) * row));
+    } else {
+        // both words of a block of 32 before the first store (268 MB with it and non-temporal stores 2.5 us more)
+        int4 p[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w)
+            if (w < words) p[w] = *reinterpret_cast<const int4*>(src + static_cast<size_t>(w) * row);
+#pragma unroll
+        for (int w = 0; w < 2; ++w)
+            if (w < words) put(w, p[w]);
     }
 }
 
@@ -168,8 +182,8 @@ __global__ void __launch_bounds__(256) dequantize_v4_kernel(const int32_t* __res
 }
 
 // Outputs or tiers that are not aligned for the wide accesses (a caller's
-// view at an odd offset, K rows that are no multiple of four channels): one
-// thread per (block, head, channel) ...
+// view at an odd offset, K rows that are no multiple of four channels), and
+// small K launches: one thread per (block, head, channel) ...
 template <typename MetaT>
 __global__ void __launch_bounds__(256) dequantize_k_kernel(const int32_t* __restrict__ packed,
                                                            const MetaT* __restrict__ scale,
@@ -226,14 +240,16 @@ int launch_quantize_k(const float* K, uint32_t* packed, void* scale, void* zero,
         const float* k = K + static_cast<size_t>(b0) * kgs * row;
         uint32_t* p = packed + static_cast<size_t>(b0) * words * row;
         const size_t m = static_cast<size_t>(b0) * row;
+        const auto launch = [&](auto kernel, auto meta) {
+            using MetaT = decltype(meta);
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, k, p, static_cast<MetaT*>(scale) + m,
+                               static_cast<MetaT*>(zero) + m, items, row, static_cast<unsigned>(D), kgs, base_dev);
+        };
+        const bool fast = !quant_one_wave(items / words);
         if (meta_fp16)
-            hipLaunchKernelGGL(quantize_k_kernel<uint16_t>, grid, dim3(256), 0, stream, k, p,
-                               static_cast<uint16_t*>(scale) + m, static_cast<uint16_t*>(zero) + m, items, row,
-                               static_cast<unsigned>(D), kgs, base_dev);
+            fast ? launch(quantize_k_kernel<uint16_t, true>, uint16_t{}) : launch(quantize_k_kernel<uint16_t, false>, uint16_t{});
         else
-            hipLaunchKernelGGL(quantize_k_kernel<float>, grid, dim3(256), 0, stream, k, p,
-                               static_cast<float*>(scale) + m, static_cast<float*>(zero) + m, items, row,
-                               static_cast<unsigned>(D), kgs, base_dev);
+            fast ? launch(quantize_k_kernel<float, true>, float{}) : launch(quantize_k_kernel<float, false>, float{});
         TT_LAUNCH_CHECK();
     }
     return TT_OK;
@@ -260,13 +276,16 @@ int launch_quantize_v(const float* V, int32_t* packed, void* scale, void* zero, 
     const long long n = static_cast<long long>(tokens) * H * group;
     if (n > kMaxThreads) TT_FAIL(TT_ERR_INVALID_ARGUMENT, "quantize_v: tokens x heads too large for one call");
     const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+    const auto launch = [&](auto kernel, auto meta) {
+        using MetaT = decltype(meta);
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, V, packed, static_cast<MetaT*>(scale),
+                           static_cast<MetaT*>(zero), tokens, H, D, group, base_dev, tokens_per_block);
+    };
+    const bool fast = !quant_one_wave(n);
     if (meta_fp16)
-        hipLaunchKernelGGL(quantize_v_kernel<uint16_t>, grid, dim3(256), 0, stream, V, packed,
-                           static_cast<uint16_t*>(scale), static_cast<uint16_t*>(zero), tokens, H, D, group, base_dev,
-                           tokens_per_block);
+        fast ? launch(quantize_v_kernel<uint16_t, true>, uint16_t{}) : launch(quantize_v_kernel<uint16_t, false>, uint16_t{});
     else
-        hipLaunchKernelGGL(quantize_v_kernel<float>, grid, dim3(256), 0, stream, V, packed, static_cast<float*>(scale),
-                           static_cast<float*>(zero), tokens, H, D, group, base_dev, tokens_per_block);
+        fast ? launch(quantize_v_kernel<float, true>, float{}) : launch(quantize_v_kernel<float, false>, float{});
     TT_LAUNCH_CHECK();
     return TT_OK;
 }
@@ -276,8 +295,8 @@ int launch_dequantize_k(const int32_t* packed, const void* scale, const void* ze
     if (num_blocks <= 0 || H * D <= 0) return TT_OK;
     const size_t meta4 = meta_fp16 ? 8 : 16;
     const long long items = static_cast<long long>(num_blocks) * (H * D / 4);
-    if (H * D % 4 == 0 && deq_k_wide_fits(items) && aligned(packed, 16) && aligned(out, 16) && aligned(scale, meta4) &&
-        aligned(zero, meta4)) {
+    if (H * D % 4 == 0 && !quant_one_wave(4 * items) && deq_k_wide_fits(items) && aligned(packed, 16) && aligned(out, 16) &&
+        aligned(scale, meta4) && aligned(zero, meta4)) {
         const dim3 grid(static_cast<unsigned>((items + 255) / 256));
         const unsigned row = static_cast<unsigned>(H * D), n = static_cast<unsigned>(items);
         const auto launch = [&](auto kernel, auto meta) {

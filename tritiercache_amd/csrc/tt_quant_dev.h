@@ -16,12 +16,26 @@ namespace tt {
 // its values instead. Without NaNs mn and mx = mn + 3 s bound every value, so
 // the quotient lies in [0, 3] and no clamp is needed. 8 instructions per value
 // instead of 17: 134 MB of V take 23.8 us against 28.9, of K 23.9 against 25.8
-// (with the flat launch).
+// (with the flat launch). FAST false divides every value at once: in a launch
+// that is over with its slowest wave, the one in fifty that does both.
 constexpr float kTieSlack = 8e-6f;
-template <int N, typename Exact>
+template <int N, bool FAST, typename Exact>
 __device__ __forceinline__ void quant_codes(const float (&x)[N], const float mn, const float s,
                                             uint32_t (&bits)[N / 16], Exact exact) {
     static_assert(N % 16 == 0, "whole words");
+    auto divide = [&] {
+#pragma unroll
+        for (int w = 0; w < N / 16; ++w) {
+            uint32_t b = 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) b |= static_cast<uint32_t>(exact(x[16 * w + i])) << (2 * i);
+            bits[w] = b;
+        }
+    };
+    if constexpr (!FAST) {
+        divide();
+        return;
+    }
     const float inv = __builtin_amdgcn_rcpf(s);
     bool slow = !(s < 1e30f);
 #pragma unroll
@@ -36,21 +50,13 @@ __device__ __forceinline__ void quant_codes(const float (&x)[N], const float mn,
         }
         bits[w] = b;
     }
-    if (slow) {
-#pragma unroll
-        for (int w = 0; w < N / 16; ++w) {
-            uint32_t b = 0;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) b |= static_cast<uint32_t>(exact(x[16 * w + i])) << (2 * i);
-            bits[w] = b;
-        }
-    }
+    if (slow) divide();
 }
 
 // K, one channel of one block (quantize_k_avx2.cpp:26-110) whose KGS values
 // are in registers. `vec` selects the 8-wide vector body semantics
 // (channel < 8*floor(D/8)) versus the scalar tail.
-template <typename MetaT, int KGS>
+template <typename MetaT, int KGS, bool FAST>
 __device__ __forceinline__ void quant_k_channel_n(const float (&x)[KGS], bool vec, MetaT* scale_dst, MetaT* zero_dst,
                                                   uint32_t (&bits)[KGS / 16]) {
     float mn = __builtin_huge_valf(), mx = -__builtin_huge_valf();
@@ -68,7 +74,7 @@ __device__ __forceinline__ void quant_k_channel_n(const float (&x)[KGS], bool ve
     const float s = vec ? x86_maxps(d3, 1e-9f) : std_max(d3, 1e-9f);
     Meta<MetaT>::store(scale_dst, 0, s);
     Meta<MetaT>::store(zero_dst, 0, mn);
-    quant_codes<KGS>(x, mn, s, bits, [&](const float v) {
+    quant_codes<KGS, FAST>(x, mn, s, bits, [&](const float v) {
         const int q = cvt_rne_i32((v - mn) / s);
         return min(max(q, 0), 3);  // the scalar tail clamps from above first: the same value
     });
@@ -78,7 +84,7 @@ __device__ __forceinline__ void quant_k_channel_n(const float (&x)[KGS], bool ve
 // `tok_stride` floats apart. Writes scale/zero and KGS/16 words spaced
 // `word_stride` apart. Every load is issued before the first use and each
 // value is read once.
-template <typename MetaT, int KGS>
+template <typename MetaT, int KGS, bool FAST>
 __device__ __forceinline__ void quant_k_channel_m(const float* __restrict__ src, size_t tok_stride, bool vec,
                                                   MetaT* scale_dst, MetaT* zero_dst, uint32_t* packed_dst,
                                                   size_t word_stride) {
@@ -86,21 +92,21 @@ __device__ __forceinline__ void quant_k_channel_m(const float* __restrict__ src,
 #pragma unroll
     for (int t = 0; t < KGS; ++t) x[t] = src[t * tok_stride];
     uint32_t bits[KGS / 16];
-    quant_k_channel_n<MetaT, KGS>(x, vec, scale_dst, zero_dst, bits);
+    quant_k_channel_n<MetaT, KGS, FAST>(x, vec, scale_dst, zero_dst, bits);
 #pragma unroll
     for (int w = 0; w < KGS / 16; ++w) packed_dst[w * word_stride] = bits[w];
 }
 
-template <typename MetaT>
+template <typename MetaT, bool FAST = true>
 __device__ __forceinline__ void quant_k_channel(const float* __restrict__ src, size_t tok_stride, int kgs, bool vec,
                                                 MetaT* scale_dst, MetaT* zero_dst, uint32_t* packed_dst,
                                                 size_t word_stride) {
     if (kgs == 16) {
-        quant_k_channel_m<MetaT, 16>(src, tok_stride, vec, scale_dst, zero_dst, packed_dst, word_stride);
+        quant_k_channel_m<MetaT, 16, FAST>(src, tok_stride, vec, scale_dst, zero_dst, packed_dst, word_stride);
         return;
     }
     if (kgs == 32) {
-        quant_k_channel_m<MetaT, 32>(src, tok_stride, vec, scale_dst, zero_dst, packed_dst, word_stride);
+        quant_k_channel_m<MetaT, 32, FAST>(src, tok_stride, vec, scale_dst, zero_dst, packed_dst, word_stride);
         return;
     }
     float mn = __builtin_huge_valf(), mx = -__builtin_huge_valf();
@@ -150,9 +156,10 @@ __device__ __forceinline__ float hmax8(const float* x) {
 }
 
 // Packs 16 channels (x[i] -> bits 2i) against the row's (mn, s).
+template <bool FAST>
 __device__ __forceinline__ uint32_t quant_v_word(const float (&x)[16], float mn, float s) {
     uint32_t bits[1];
-    quant_codes<16>(x, mn, s, bits, [&](const float v) {
+    quant_codes<16, FAST>(x, mn, s, bits, [&](const float v) {
         const int q = cvt_rne_i32((v - mn) / s);
         return max(min(q, 3), 0);
     });
@@ -172,7 +179,7 @@ __device__ __forceinline__ uint32_t quant_v_word(const float (&x)[16], float mn,
 // always the lower channels': the same value as the reference's fold, bit
 // for bit. Padding lanes hold +inf / -inf, which a real lane's value always
 // keeps (a tie with +inf keeps the lower lane's +inf, the same value).
-template <typename MetaT>
+template <typename MetaT, bool FAST = true>
 __device__ __forceinline__ void quant_v_row_lanes(const float* __restrict__ v, int w, int wpr, int group,
                                                   MetaT* scale_dst, MetaT* zero_dst, int32_t* packed_dst) {
     const bool real = w < wpr;
@@ -209,7 +216,7 @@ __device__ __forceinline__ void quant_v_row_lanes(const float* __restrict__ v, i
         Meta<MetaT>::store(scale_dst, 0, s);
         Meta<MetaT>::store(zero_dst, 0, mn);
     }
-    if (real) packed_dst[w] = static_cast<int32_t>(quant_v_word(x, mn, s));
+    if (real) packed_dst[w] = static_cast<int32_t>(quant_v_word<FAST>(x, mn, s));
 }
 
 // The same row on one thread, for rows of more than 64 words: the
@@ -232,7 +239,7 @@ __device__ __forceinline__ void quant_v_row_serial(const float* __restrict__ v, 
         float x[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] = v[16 * w + i];
-        packed_dst[w] = static_cast<int32_t>(quant_v_word(x, mn, s));
+        packed_dst[w] = static_cast<int32_t>(quant_v_word<true>(x, mn, s));
     }
 }
 

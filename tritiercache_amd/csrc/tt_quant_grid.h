@@ -14,6 +14,14 @@ inline int quant_k_slice(const int num_blocks, const long long row) {
     return static_cast<int>(std::min<long long>(num_blocks, kMaxThreads / row));
 }
 
+// Launches of at most a wave per SIMD (256 CUs of four; K in blocks of 32, whose
+// lanes hold twice the values: two) are over with their slowest wave: there the
+// quantisers divide every value (K in blocks of 16, 2 MB, 3.4 us against 3.6 with
+// the reciprocal codes, 5 MB 4.0 against 3.7; in blocks of 32, 2 MB 4.6 against
+// 5.8, 10 MB 5.8 against 6.3, 20 MB 7.1 against 6.8; V, 2 MB 3.6 against 3.7, 5 MB
+// 4.0 against 3.8).
+inline bool quant_one_wave(const long long threads) { return threads <= 4 * 256 * 64; }
+
 // The wide K dequantiser holds four channels per thread.
 inline bool deq_k_wide_fits(const long long quads) { return quads <= kMaxThreads; }
 
