@@ -190,3 +190,26 @@ def test_workspace_size_query_validates_like_the_entry_points():
     p = 0x10000
     rc = L.tt_attention_partials(p, p, p, 1 << 30, p, p, p, p, p, p, p, 1 << 26, 64, 8, 128, 32, 0, 0, p, 1 << 40, None)
     assert rc == 1 and "2^31" in _lib.last_error()
+
+
+def test_workspace_size_covers_every_shorter_context():
+    """No call of at most the queried counts is refused for its workspace. Without a device an accepted call ends at
+    its launch (TT_ERR_HIP); with one it would run on the placeholder pointers, so this is a test for the CPU."""
+    import random
+
+    from tritiercache_amd import _lib
+
+    L = _lib.load()
+    if L.tt_device_count() > 0:
+        pytest.skip("placeholder pointers: only where no kernel can run")
+    rng, p = random.Random(5), 0x10000
+    for _ in range(8000):
+        hkv, g = rng.choice((1, 2, 3, 4, 7, 8, 10, 16, 32, 40, 64, 128)), rng.choice((1, 2, 3, 4, 7, 8, 12))
+        d, kgs, w = rng.choice((128, 128, 64, 64, 16, 80, 144, 256)), rng.choice((16, 32)), rng.randint(0, 1)
+        nd, nb = rng.choice((0, 1, 16, 300, 3000)) + rng.randint(0, 40), int(10 ** rng.uniform(0, 4.2))
+        size = L.tt_fused_attention_workspace_bytes(nd, nb, hkv * g, hkv, d, kgs, w)
+        for a, b in ((nd, nb), (nd, rng.randint(0, nb)), (rng.randint(0, nd), nb), (0, rng.randint(1, nb))):
+            if size and a + b > 0:
+                rc = L.tt_attention_partials(p, p, p, a, p, p, p, p, p, p, p, b, hkv * g, hkv, d, kgs,
+                                             rng.randint(0, 1), w, p, size, None)
+                assert rc == 5, ((nd, nb), (a, b), hkv * g, hkv, d, kgs, w, _lib.last_error())

@@ -7,6 +7,7 @@
 // kernels (GQA ratio integral, head_dim a multiple of 16 of at most 256).
 #include "tt_attn.h"
 
+#include <algorithm>
 #include <mutex>
 #include <unordered_map>
 
@@ -27,7 +28,9 @@ struct DeviceWorkspace {
 std::mutex g_ws_mutex;
 std::unordered_map<int, DeviceWorkspace> g_ws;
 
-int get_workspace(size_t bytes, void** out) {
+// `reserve`: the size to grow to where the workspace is smaller than `bytes`.
+template <typename Reserve>
+int get_workspace(size_t bytes, Reserve reserve, void** out) {
     int dev = 0;
     TT_HIP_CHECK(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(g_ws_mutex);
@@ -39,7 +42,7 @@ int get_workspace(size_t bytes, void** out) {
             w.ptr = nullptr;
             w.bytes = 0;
         }
-        const size_t nb = std::max(bytes, static_cast<size_t>(1) << 20);
+        const size_t nb = std::max({bytes, static_cast<size_t>(reserve()), static_cast<size_t>(1) << 20});
         TT_HIP_CHECK(hipMalloc(&w.ptr, nb));
         w.bytes = nb;
     }
@@ -141,8 +144,10 @@ int fused_impl(const float* Q, const float* dK, const float* dV, int dense_count
     if (phase == kFinalize && mw && !logits)
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "mean_attn_weights requested but the partials were planned without them.");
     if (own_ws) {
-        // for every shorter context too: a call captured after a longer one allocates nothing
-        rc = get_workspace(attn_workspace_bytes(dense_count, num_blocks, Hq, Hkv, D, kgs, logits, meta_fp16), &ws);
+        // grown for every shorter context too: a call captured after a longer one allocates nothing
+        rc = get_workspace(
+            plan.bytes,
+            [&] { return attn_workspace_bytes(dense_count, num_blocks, Hq, Hkv, D, kgs, logits, meta_fp16); }, &ws);
         if (rc) return rc;
     } else if (!ws || ws_bytes < plan.bytes) {
         TT_FAIL(TT_ERR_INVALID_ARGUMENT, "workspace is NULL or smaller than tt_fused_attention_workspace_bytes().");
